@@ -321,16 +321,98 @@ template <> MF_HD V<4> mul_dbl<4>(const V<4> &a, double d) {
 
 // Long division: N+1 partial quotients q_i = r0 / y0, the remainder updated
 // as r - y*q_i with the N-limb x binary64 product, then an error-free
-// renormalisation of the quotient digits.
+// renormalisation of the quotient digits. A wave's time in a serial chain is
+// its instruction count (four cycles each; a dependent binary64 instruction
+// waits for nothing more), so the loop is unrolled: left to itself the
+// compiler keeps the four-limb one rolled and selects each digit's register
+// by compares (4456 cycles a division, unrolled 3560; two and three limbs
+// 568 and 1712 either way). One reciprocal for all quotients was measured
+// too: 572 / 1444 / 3464 cycles with the range check it needs, and twice
+// that where a remainder vanishes and the check fails.
 template <int N> MF_HD V<N> div(const V<N> &x, const V<N> &y) {
     if constexpr (N == 1) {
         V<1> r; r.x[0] = x.x[0] / y.x[0]; return r;
     } else {
         double q[N + 1];
         V<N> r = x;
+#pragma unroll
         for (int i = 0; i <= N; ++i) {
             q[i] = r.x[0] / y.x[0];
             if (i < N) r = sub(r, mul_dbl<N>(y, q[i]));
+        }
+        return renorm_np1<N>(q);
+    }
+}
+
+// x - (p, e, 0, ..): add(x, neg(.)) without the operations whose result is
+// known (a sum with a zero; the remaining "+ 0.0" keep the sign a zero gets).
+MF_HD V<3> sub_two(const V<3> &x, double p, double e0) {
+    double a, b, c, d, e = x.x[2];
+    two_sum(x.x[0], -p, a, b);
+    two_sum(x.x[1], -e0, c, d);
+    fast_two_sum(a, c, a, c);
+    two_sum(d, e, d, e);
+    fast_two_sum(a, d, a, d);
+    two_sum(b, c, b, c);
+    c += e;
+    two_sum(c, d, c, d);
+    two_sum(b, c, b, c);
+    fast_two_sum(a, b, a, b);
+    c += d;
+    fast_two_sum(b, c, b, c);
+    fast_two_sum(a, b, a, b);
+    fast_two_sum(b, c, b, c);
+    V<3> r; r.x[0] = a; r.x[1] = b; r.x[2] = c; return r;
+}
+MF_HD V<4> sub_two(const V<4> &x, double p, double e0) {
+    double a, b, c, d, e = x.x[2], f = x.x[3] + 0.0;
+    two_sum(x.x[0], -p, a, b);
+    two_sum(x.x[1], -e0, c, d);
+    fast_two_sum(a, c, a, c);
+    two_sum(d, e, d, e);
+    fast_two_sum(c, d, c, d);
+    two_sum(e, f, e, f);
+    fast_two_sum(a, c, a, c);
+    fast_two_sum(d, e, d, e);
+    two_sum(b, d, b, d);
+    c += 0.0;
+    e += f;
+    two_sum(b, c, b, c);
+    two_sum(d, e, d, e);
+    fast_two_sum(a, b, a, b);
+    two_sum(c, d, c, d);
+    e += 0.0;
+    fast_two_sum(b, c, b, c);
+    two_sum(d, e, d, e);
+    fast_two_sum(a, b, a, b);
+    fast_two_sum(c, d, c, d);
+    fast_two_sum(b, c, b, c);
+    d += e;
+    fast_two_sum(a, b, a, b);
+    fast_two_sum(c, d, c, d);
+    fast_two_sum(b, c, b, c);
+    fast_two_sum(c, d, c, d);
+    V<4> r; r.x[0] = a; r.x[1] = b; r.x[2] = c; r.x[3] = d; return r;
+}
+
+// x / (s, 0, ..), x and s positive, with div's bits (the first Heron step's
+// divisor has one limb): y * q_i is then TwoProd(s, q_i), 2 operations for 46
+// (four limbs), and the remainder's update 95 for 124 (one wave's sqrt, with
+// the unrolled division: x4 9220 -> 6780 cycles, x3 4316 -> 3464).
+template <int N> MF_HD V<N> div_lead(const V<N> &x, double s) {
+    if constexpr (N < 3) {
+        return div(x, from<N>(s));
+    } else {
+        double q[N + 1];
+        V<N> r = x;
+#pragma unroll
+        for (int i = 0; i <= N; ++i) {
+            q[i] = r.x[0] / s;
+            if (i < N) {
+                double p, e;
+                two_prod(s, q[i], p, e);
+                r = sub_two(r, p, e);
+            }
         }
         return renorm_np1<N>(q);
     }
@@ -343,8 +425,9 @@ template <int N> MF_HD V<N> sqrt(const V<N> &x) {
     }
     V<N> s = from<N>(::sqrt(x.x[0]));
     constexpr int iters = N == 1 ? 0 : (N == 2 ? 1 : 2);
+#pragma unroll
     for (int it = 0; it < iters; ++it) {
-        s = add(s, div(x, s));
+        s = add(s, it == 0 ? div_lead(x, s.x[0]) : div(x, s));
         for (int i = 0; i < N; ++i) s.x[i] *= 0.5;
     }
     return s;
