@@ -18,7 +18,7 @@
 // Backward substitution with MFLA's ascending-q chain has an O(n^2) serial
 // dependency per right-hand side (row p's first term needs X(p+1), the last
 // unknown solved). Two orders are provided: the exact MFLA order
-// (k_trsm_seq, one thread per right-hand side) and a blocked right-looking
+// (k_trsm_chain_bwd) and a blocked right-looking
 // order (descending blocks) whose rounding differs from MFLA's but stays
 // within the same c*n*u bound.
 #include <type_traits>
@@ -293,19 +293,94 @@ __global__ __launch_bounds__(256) void k_trsm_side_wait(const unsigned *start_si
     for (int64_t e = threadIdx.x; e < rows * nrhs; e += blockDim.x) stv<N>(X, r0 + e % rows, e / rows, bad);
 }
 
-// Exact MFLA order for backward substitution: one thread per right-hand side.
-template <int N>
-__global__ void k_trsm_seq_bwd(int64_t n, int64_t nrhs, DV X, DV CA, DV D, int unit, int swap, const Status *st, int64_t lim) {
+// Exact MFLA order for backward substitution. Row p's chain starts with
+// X(p + 1), the unknown solved last, so a right-hand side is one serial chain
+// of n^2 / 2 terms whose time is its wave's instruction count. Only the
+// additions have to be on it: wave 0 of a workgroup runs the chains of R
+// right-hand sides (a lane each), the three other waves form the negated
+// products CA(p, q) X(q) of the next CH terms in LDS meanwhile (one buffer is
+// read while the other is filled, a barrier per CH terms). The chain wave
+// itself forms the product with X(p + 1), which no one else can have yet; the
+// next row's first products need X down to p + 1 only. Per element the
+// operations and their order are MFLA's, msub(v, a, x) = v + (-(a x)).
+// R: 1 up to 256 right-hand sides (a chain wave per CU), 16 up to 4096 and 64
+// beyond keep it at that (one lane per CU has the same speed as 64).
+// x4, n = 256, one right-hand side: 17.5 ms with every
+// term's product on the chain -> 7.6 ms (32640 additions at ~570 cycles).
+template <int N, int R>
+__global__ __launch_bounds__(256) void k_trsm_chain_bwd(int64_t n, int64_t nrhs, DV X, DV CA, DV D, int unit, int swap, const Status *st,
+                                                        int64_t lim) {
     if (st && st->info != 0 && (lim == 0 || st->info < 0 || st->info <= lim)) return;
-    const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= nrhs) return;
-    for (int64_t p = n - 1; p >= 0; --p) {
-        mf::V<N> v = ld<N>(X, p, c);
-        for (int64_t q = p + 1; q < n; ++q)
-            v = swap ? mf::msub(v, ld<N>(X, q, c), ld<N>(CA, p, q)) : mf::msub(v, ld<N>(CA, p, q), ld<N>(X, q, c));
-        if (!unit) v = mf::div(v, ld<N>(D, p, p));
-        stv<N>(X, p, c, v);
+    constexpr int CH = R == 1 ? 192 : (R == 16 ? 24 : 9);   // CH * R terms: 1, 2 or 3 per producer thread
+    constexpr int LD = CH * N + 2;                          // a lane's terms, 16-byte aligned, spread over the banks
+    __shared__ __align__(16) double buf[2][R * LD];
+    const int t = threadIdx.x;
+    const bool chain = t < 64;
+    const int r = t % R;
+    const int64_t c0 = (int64_t)blockIdx.x * R, c = c0 + r, cc = c < nrhs ? c : nrhs - 1;
+    auto produce = [&](double *to, int64_t p, int64_t q0) {
+        for (int e = t - 64; e < CH * R; e += 192) {
+            const int qi = e % CH, rr = e / CH;
+            const int64_t q = q0 + qi, cx = c0 + rr < nrhs ? c0 + rr : nrhs - 1;
+            if (q >= n) continue;
+            const mf::V<N> a = ld<N>(CA, p, q), x = ld<N>(X, q, cx);
+            lds_put<N>(to + rr * LD + qi * N, mf::neg(swap ? mf::mul(x, a) : mf::mul(a, x)));
+        }
+    };
+    // the chain wave's operands of the row to come: X(p), CA(p, p + 1), D(p, p)
+    mf::V<N> v = mf::zero<N>(), xn = mf::zero<N>(), an = mf::zero<N>(), dn = mf::zero<N>();
+    if (chain) {
+        xn = ld<N>(X, n - 1, cc);
+        if (!unit) dn = ld<N>(D, n - 1, n - 1);
     }
+    int b = 0;
+    for (int64_t p = n - 1; p >= 0; --p) {
+        const int64_t terms = n - p - 2;                     // after the first
+        const int64_t chunks = terms > CH ? (terms + CH - 1) / CH : 1;
+        mf::V<N> d = mf::zero<N>();
+        for (int64_t i = 0; i < chunks; ++i) {
+            if (chain) {
+                if (i == 0) {
+                    const mf::V<N> xp = v, a = an;
+                    v = xn;
+                    d = dn;
+                    if (p > 0) {
+                        xn = ld<N>(X, p - 1, cc);
+                        an = ld<N>(CA, p - 1, p);
+                        if (!unit) dn = ld<N>(D, p - 1, p - 1);
+                    }
+                    if (p + 1 < n) v = swap ? mf::msub(v, xp, a) : mf::msub(v, a, xp);
+                }
+                const int64_t left = terms - i * CH;
+                const int m = left > CH ? CH : (left > 0 ? (int)left : 0);
+                const double *from = &buf[b][r * LD];
+                v = add_terms<N, CH>(v, m, [&](int k) { return lds_get<N>(from + k * N); });
+                if (i == chunks - 1) {
+                    if (!unit) v = mf::div(v, d);
+                    if (t < R && c < nrhs) stv<N>(X, p, c, v);
+                }
+            } else if (i + 1 < chunks) {
+                produce(buf[b ^ 1], p, p + 2 + (i + 1) * CH);
+            } else if (p > 0) {
+                produce(buf[b ^ 1], p - 1, p + 1);
+            }
+            __syncthreads();
+            b ^= 1;
+        }
+    }
+}
+
+template <int N>
+static hipError_t chain_bwd(hipStream_t s, const TrsmArgs &a, const DV &X, const DV &CA, const DV &D, const Status *st) {
+    auto launch = [&](auto rtag) {
+        constexpr int R = decltype(rtag)::value;
+        hipLaunchKernelGGL((k_trsm_chain_bwd<N, R>), dim3((unsigned)cdiv(a.nrhs, R)), dim3(256), 0, s, a.n, a.nrhs, X, CA, D, a.unit,
+                           a.swap_product, st, a.status_limit);
+    };
+    if (a.nrhs <= 256) launch(std::integral_constant<int, 1>());
+    else if (a.nrhs <= 4096) launch(std::integral_constant<int, 16>());
+    else launch(std::integral_constant<int, 64>());
+    return hipGetLastError();
 }
 
 static DV sub(const DV &v, int64_t i, int64_t j) { return DV{v.p + i * v.rs + j * v.cs, v.rs, v.cs, v.ls}; }
@@ -539,10 +614,7 @@ static hipError_t solve_t(hipStream_t s, const TrsmArgs &a, const DV &X, const D
         }
         return hipSuccess;
     }
-    if (a.exact_order) {
-        hipLaunchKernelGGL(k_trsm_seq_bwd<N>, dim3((unsigned)cdiv(nrhs, 64)), dim3(64), 0, s, n, nrhs, X, CA, D, a.unit, a.swap_product, st, a.status_limit);
-        return hipGetLastError();
-    }
+    if (a.exact_order) return chain_bwd<N>(s, a, X, CA, D, st);
     for (int64_t p1 = n; p1 > 0; p1 -= TB) {
         const int64_t p0 = p1 > TB ? p1 - TB : 0;
         const int nbk = (int)(p1 - p0);

@@ -88,6 +88,30 @@ __device__ inline bool wait_flag(const unsigned *flag, unsigned value) {
     return true;
 }
 
+// acc + term(0) + term(1) + ... + term(m - 1) in that order, 0 <= m <= CH: a
+// chain's additions, its terms (in LDS) read a group of four ahead and a
+// branch taken once a group. term(k) is read for any k < CH.
+template <int N, int CH, typename T> __device__ __forceinline__ mf::V<N> add_terms(mf::V<N> acc, int m, const T &term) {
+    constexpr int G = 4;
+    mf::V<N> next[G];
+#pragma unroll
+    for (int g = 0; g < G; ++g) next[g] = term(g < CH ? g : CH - 1);
+    int k = 0;
+    for (; k + G <= m; k += G) {
+        mf::V<N> now[G];
+        const int ahead = k + 2 * G <= CH ? k + G : CH - G;
+#pragma unroll
+        for (int g = 0; g < G; ++g) {
+            now[g] = next[g];
+            next[g] = term(ahead + g);
+        }
+#pragma unroll
+        for (int g = 0; g < G; ++g) acc = mf::add(acc, now[g]);
+    }
+    for (; k < m; ++k) acc = mf::add(acc, term(k));
+    return acc;
+}
+
 inline int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
 }  // namespace mfk
