@@ -109,56 +109,87 @@ __global__ void k_arith(int op, int64_t count, const double *x, const double *y,
 }
 
 // --------------------------------------------------------------- GEMV
-// src/kernels/gemv.jl:1-93: one thread per output, ascending reduction. The
-// reduction is one serial chain per output (MFLA's order), so the kernel is
-// bound by the chain's latency, not by HBM: 64-thread workgroups spread the
-// outputs over as many CUs as possible, and a ring of GV_PF prefetched
-// (A, x) pairs keeps the loads GV_PF steps ahead of the chain.
-constexpr int GV_PF = 8;
+// src/kernels/gemv.jl:1-93, src/kernels/symv.jl:1-36: each output is one
+// ascending chain acc = acc + a(o, k) x(k) (symv: every column in order, read
+// from the authoritative triangle). The chain is MFLA's order, so a kernel
+// cannot be shorter than `red` additions of one wave (124 instructions for
+// four limbs, four cycles each); the products and the loads need not be on
+// it. Wave 0 of a workgroup adds for O outputs (a lane each), three waves
+// form the next CH columns' products in LDS from operands they loaded a chunk
+// earlier. O = 16 while that gives at most two workgroups per CU (a wave of
+// 16 chains takes as long as one of 64, and four times as many CUs load), else
+// 64. x4 4096 x 4096: 2.44 ms with
+// product and addition in one thread -> 0.97 ms (566 cycles a column).
+// SYM 0: A(o, k) through the view (transposed: the lanes run along k); 1 / 2:
+// symmetric with the lower / upper triangle read. Y and X: a column per
+// blockIdx.y.
+constexpr int GV_ITEMS = 4;   // products per producer thread and chunk
 
-template <int N>
-__global__ __launch_bounds__(64) void k_gemv(int trans, int64_t outs, int64_t red, DV A, DV x, DV y, S<N> alpha, S<N> beta,
-                                             int beta_zero, const Status *st) {
+template <int N, int O, int SYM>
+__global__ __launch_bounds__(256) void k_matvec(int64_t outs, int64_t red, DV A, DV X, DV Y, S<N> alpha, S<N> beta, int beta_zero,
+                                                const Status *st) {
     if (st && st->info != 0) return;
-    const int64_t o = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (o >= outs) return;
-    const DV Ao = trans ? DV{A.p + o * A.cs, A.cs, A.rs, A.ls} : DV{A.p + o * A.rs, A.rs, A.cs, A.ls};   // Ao(0, k)
-    mf::V<N> acc = mf::zero<N>();
-    mf::V<N> ra[GV_PF], rx[GV_PF];
+    constexpr int CH = 192 * GV_ITEMS / O, LD = N * O + 2;
+    __shared__ double buf[2][CH * LD];
+    const int t = threadIdx.x;
+    const int64_t o0 = (int64_t)blockIdx.x * O, col = blockIdx.y;
+    const int64_t chunks = (red + CH - 1) / CH;
+    if (t >= 64) {
+        // item q of this thread: output io[q] (clamped into the operand), k0 + ik[q]
+        const bool kfast = SYM == 0 && A.cs == 1 && A.rs != 1;
+        mf::V<N> a[GV_ITEMS], x[GV_ITEMS];
+        auto place = [&](int q, int &o, int &k) {
+            const int e = t - 64 + 192 * q;
+            if (kfast) { k = e % CH; o = e / CH; } else { o = e % O; k = e / O; }
+        };
+        auto fetch = [&](int64_t k0) {
 #pragma unroll
-    for (int q = 0; q < GV_PF; ++q) {
-        if (q < red) { ra[q] = ld<N>(Ao, 0, q); rx[q] = ld<N>(x, q, 0); }
-    }
-    int64_t k = 0;
-    for (; k + GV_PF <= red; k += GV_PF) {
+            for (int q = 0; q < GV_ITEMS; ++q) {
+                int o, kk;
+                place(q, o, kk);
+                const int64_t i = o0 + o < outs ? o0 + o : outs - 1, k = k0 + kk < red ? k0 + kk : red - 1;
+                const bool other = (SYM == 1 && k > i) || (SYM == 2 && k < i);
+                a[q] = other ? ld<N>(A, k, i) : ld<N>(A, i, k);
+                x[q] = ld<N>(X, k, col);
+            }
+        };
+        if (chunks > 0) fetch(0);
+        for (int64_t ch = 0; ch <= chunks; ++ch) {
+            if (ch < chunks) {
+                double *to = buf[ch & 1];
+                mf::V<N> p[GV_ITEMS];
 #pragma unroll
-        for (int q = 0; q < GV_PF; ++q) {
-            acc = mf::mac(acc, ra[q], rx[q]);
-            const int64_t kn = k + GV_PF + q;
-            if (kn < red) { ra[q] = ld<N>(Ao, 0, kn); rx[q] = ld<N>(x, kn, 0); }
+                for (int q = 0; q < GV_ITEMS; ++q) p[q] = mf::mul(a[q], x[q]);
+                if (ch + 1 < chunks) fetch((ch + 1) * CH);
+#pragma unroll
+                for (int q = 0; q < GV_ITEMS; ++q) {
+                    int o, kk;
+                    place(q, o, kk);
+#pragma unroll
+                    for (int l = 0; l < N; ++l) to[kk * LD + l * O + o] = p[q].x[l];
+                }
+            }
+            __syncthreads();
         }
+        return;
     }
-#pragma unroll
-    for (int q = 0; q < GV_PF; ++q)
-        if (k + q < red) acc = mf::mac(acc, ra[q], rx[q]);
-    mf::V<N> r = beta_zero ? mf::mul(sv(alpha), acc) : mf::add(mf::mul(sv(alpha), acc), mf::mul(sv(beta), ld<N>(y, o, 0)));
-    stv<N>(y, o, 0, r);
-}
-
-// src/kernels/symv.jl:1-36: columns 1..row-1, diagonal, row+1..n, reading
-// only the authoritative triangle. One thread per output row.
-template <int N>
-__global__ __launch_bounds__(256) void k_symv(int upper, int64_t n, DV A, DV X, DV Y, int64_t nrhs, S<N> alpha, S<N> beta,
-                                              int beta_zero) {
-    const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= n * nrhs) return;
-    const int64_t row = e % n, c = e / n;
+    const int o = t % O;
     mf::V<N> acc = mf::zero<N>();
-    for (int64_t col = 0; col < row; ++col) acc = mf::mac(acc, upper ? ld<N>(A, col, row) : ld<N>(A, row, col), ld<N>(X, col, c));
-    acc = mf::mac(acc, ld<N>(A, row, row), ld<N>(X, row, c));
-    for (int64_t col = row + 1; col < n; ++col) acc = mf::mac(acc, upper ? ld<N>(A, row, col) : ld<N>(A, col, row), ld<N>(X, col, c));
-    mf::V<N> r = beta_zero ? mf::mul(sv(alpha), acc) : mf::add(mf::mul(sv(alpha), acc), mf::mul(sv(beta), ld<N>(Y, row, c)));
-    stv<N>(Y, row, c, r);
+    for (int64_t ch = 0; ch <= chunks; ++ch) {
+        if (ch > 0) {
+            const double *from = buf[(ch - 1) & 1] + o;
+            const int64_t left = red - (ch - 1) * CH;
+            const int m = left < CH ? (int)left : CH;
+            auto term = [&](int k) { mf::V<N> v; _Pragma("unroll") for (int l = 0; l < N; ++l) v.x[l] = from[k * LD + l * O]; return v; };
+            acc = add_terms<N, CH>(acc, m, term);
+        }
+        __syncthreads();
+    }
+    if (t < O && o0 + o < outs) {
+        const int64_t i = o0 + o;
+        const mf::V<N> r = beta_zero ? mf::mul(sv(alpha), acc) : mf::add(mf::mul(sv(alpha), acc), mf::mul(sv(beta), ld<N>(Y, i, col)));
+        stv<N>(Y, i, col, r);
+    }
 }
 
 // ------------------------------------------------- mixed residual
@@ -324,20 +355,36 @@ hipError_t finite_check(int N, hipStream_t s, int64_t m, int64_t n, const DV &A,
     return hipGetLastError();
 }
 
+template <int N, int SYM>
+static void matvec(hipStream_t s, int64_t outs, int64_t red, int64_t nrhs, const DV &A, const DV &X, const DV &Y, const double *alpha,
+                   const double *beta, int beta_zero, const Status *st) {
+    const bool narrow = cdiv(outs, 16) * nrhs <= 512;
+    for (int64_t c0 = 0; c0 < nrhs; c0 += 65535) {   // grid.y's limit
+        const unsigned nc = (unsigned)(nrhs - c0 < 65535 ? nrhs - c0 : 65535);
+        const DV Xc{X.p + c0 * X.cs, X.rs, X.cs, X.ls}, Yc{Y.p + c0 * Y.cs, Y.rs, Y.cs, Y.ls};
+        if (narrow)
+            hipLaunchKernelGGL((k_matvec<N, 16, SYM>), dim3((unsigned)cdiv(outs, 16), nc), dim3(256), 0, s, outs, red, A, Xc, Yc, mk<N>(alpha),
+                               mk<N>(beta), beta_zero, st);
+        else
+            hipLaunchKernelGGL((k_matvec<N, 64, SYM>), dim3((unsigned)cdiv(outs, 64), nc), dim3(256), 0, s, outs, red, A, Xc, Yc, mk<N>(alpha),
+                               mk<N>(beta), beta_zero, st);
+    }
+}
+
 hipError_t gemv(int N, hipStream_t s, int trans, int64_t m, int64_t n, const DV &A, const DV &x, const DV &y, const double *alpha,
                 const double *beta, int beta_zero, const Status *st) {
     const int64_t outs = trans ? n : m, red = trans ? m : n;
     if (outs == 0) return hipSuccess;
-    MF_DISPATCH(N, hipLaunchKernelGGL(k_gemv<NN>, dim3((unsigned)((outs + 63) / 64)), dim3(64), 0, s, trans, outs, red, A, x, y, mk<NN>(alpha),
-                                      mk<NN>(beta), beta_zero, st));
+    const DV Ao = trans ? DV{A.p, A.cs, A.rs, A.ls} : A;   // Ao(o, k)
+    MF_DISPATCH(N, (matvec<NN, 0>(s, outs, red, 1, Ao, x, y, alpha, beta, beta_zero, st)));
     return hipGetLastError();
 }
 
 hipError_t symv(int N, hipStream_t s, int upper, int64_t n, int64_t nrhs, const DV &A, const DV &X, const DV &Y, const double *alpha,
                 const double *beta, int beta_zero) {
     if (n * nrhs == 0) return hipSuccess;
-    MF_DISPATCH(N, hipLaunchKernelGGL(k_symv<NN>, dim3(nb256(n * nrhs)), dim3(256), 0, s, upper, n, A, X, Y, nrhs, mk<NN>(alpha),
-                                      mk<NN>(beta), beta_zero));
+    if (upper) MF_DISPATCH(N, (matvec<NN, 2>(s, n, n, nrhs, A, X, Y, alpha, beta, beta_zero, nullptr)))
+    else MF_DISPATCH(N, (matvec<NN, 1>(s, n, n, nrhs, A, X, Y, alpha, beta, beta_zero, nullptr)));
     return hipGetLastError();
 }
 
