@@ -291,26 +291,24 @@ int ozaki_gemm(mfla_handle h, int N, int64_t m, int64_t n, int64_t k, const DV &
                const double *beta) {
     const int64_t al = mfk::oz_row_align(), ld = (k + al - 1) / al * al;
     if (ld > 8192) return fail(MFLA_ERR_ARGUMENT, "gemm_strategy=:ozaki supports reduction lengths up to 8192");
-    const int S = mfk::oz_digits(N), U = S;
+    const int S = mfk::oz_gemm_digits(N, ld);
     const int64_t mx = std::max(m, n);
     size_t off = 0;
     auto take = [&](size_t bytes) { size_t o = off; off += (bytes + 255) / 256 * 256; return o; };
     const size_t o_ea = take(sizeof(int) * m), o_eb = take(sizeof(int) * n), o_part = take(sizeof(double) * mfk::oz_chunks() * mx);
-    const size_t o_da = take((size_t)S * m * ld), o_db = take((size_t)S * n * ld), o_pl = take(sizeof(int32_t) * (size_t)(U + 1) * m * n);
+    const size_t o_da = take(mfk::oz_bytes(m, ld, S)), o_db = take(mfk::oz_bytes(n, ld, S));
     char *base = (char *)grow_scratch(h, off);
     if (!base) return fail(MFLA_ERR_HIP, "scratch allocation failed (%zu bytes)", off);
     int *ea = (int *)(base + o_ea), *eb = (int *)(base + o_eb);
     double *part = (double *)(base + o_part);
     int8_t *da = (int8_t *)(base + o_da), *db = (int8_t *)(base + o_db);
-    int32_t *pl = (int32_t *)(base + o_pl);
     hipStream_t s = h->stream;
     const DV Bt{B.p, B.cs, B.rs, B.ls};                 // Bt(j, kk) = B(kk, j)
     HIPCHK(mfk::oz_exponents(s, m, k, A, 0, ea, part));
     HIPCHK(mfk::oz_exponents(s, n, k, Bt, 0, eb, part));
-    HIPCHK(mfk::oz_split(N, s, m, k, A, 0, ea, S, da, ld, (int64_t)m * ld));
-    HIPCHK(mfk::oz_split(N, s, n, k, Bt, 0, eb, S, db, ld, (int64_t)n * ld));
-    HIPCHK(mfk::oz_gemm(s, m, n, ld, da, ld, (int64_t)m * ld, S, db, ld, (int64_t)n * ld, S, U, pl));
-    HIPCHK(mfk::oz_combine(N, s, m, n, U, pl, ea, eb, C, alpha, beta, scalar_is_zero(beta, N) ? 1 : 0, 0));
+    HIPCHK(mfk::oz_split(N, s, m, k, A, 0, ea, S, da, ld));
+    HIPCHK(mfk::oz_split(N, s, n, k, Bt, 0, eb, S, db, ld));
+    HIPCHK(mfk::oz_gemm(N, s, m, n, ld, S, da, db, ea, eb, C, alpha, beta, scalar_is_zero(beta, N) ? 1 : 0));
     return MFLA_OK;
 }
 
@@ -1769,13 +1767,13 @@ struct RefineWs {
     double *F, *Inv, *InvU, *Y, *D, *R, *P, *rows, *part, *stats;
     int64_t *perm, *ipiv;
     int64_t ksplit;
-    // Ozaki residual: digit planes of A (S planes of planeA bytes in the
-    // fragment layout), of the correction (T x nrhs x ld int8), exponents,
+    // Ozaki residual: digit planes of A (S in the fragment
+    // layout), of the correction (T x nrhs x ld int8), exponents,
     // int32 digit-pair sums
     int8_t *dA, *dD;
     int *eA, *eD;
     int32_t *planes;
-    int64_t ld, planeA;
+    int64_t ld;
     int S, T;
 };
 constexpr int kOzCorrectionDigits = 6;   // = mfk::oz_narrow_digits()
@@ -1815,8 +1813,7 @@ int64_t refine_layout(int N, int kind, int64_t n, int64_t nrhs, double *base, Re
         w.ld = (n + mfk::oz_row_align() - 1) / mfk::oz_row_align() * mfk::oz_row_align();
         w.S = mfk::oz_digits(N);
         w.T = kOzCorrectionDigits;
-        w.planeA = (n + 15) / 16 * 16 * w.ld;   // fragment layout: rows padded to 16
-        w.dA = (int8_t *)take((w.S * w.planeA + 7) / 8);
+        w.dA = (int8_t *)take((mfk::oz_bytes(n, w.ld, w.S) + 7) / 8);
         w.dD = (int8_t *)take((w.T * nrhs * w.ld + 7) / 8);
         w.eA = (int *)take((n + 1) / 2);
         w.eD = (int *)take((nrhs + 1) / 2);
@@ -2023,7 +2020,7 @@ int mfla_refine_solve(mfla_handle h, int N, int kind_flags, int uplo, mfla_matri
     for (double v : hrows) anorm = std::max(anorm, v);
     if (ozaki) {   // A's digit planes, once per solve
         HIPCHK(mfk::oz_exponents(s, n, n, Ahi, kernel_uplo(uplo), w.eA, w.part));
-        HIPCHK(mfk::oz_split(N, s, n, n, Ahi, kernel_uplo(uplo), w.eA, w.S, w.dA, w.ld, w.planeA, true));
+        HIPCHK(mfk::oz_split(N, s, n, n, Ahi, kernel_uplo(uplo), w.eA, w.S, w.dA, w.ld));
     }
     clk.mark(ST_FACTOR);
 
@@ -2061,8 +2058,8 @@ int mfla_refine_solve(mfla_handle h, int N, int kind_flags, int uplo, mfla_matri
             HIPCHK(mfk::add_mixed(1, N, s, n, nrhs, dvn(X), D));
             clk.mark(ST_UPDATE);
             const int U = w.S + w.T - 2;
-            HIPCHK(mfk::oz_gemm_narrow(s, n, nrhs, w.ld, w.dA, w.planeA, w.S, w.dD, w.ld, nrhs * w.ld, w.planes));
-            HIPCHK(mfk::oz_combine(N, s, n, nrhs, U, w.planes, w.eA, w.eD, R, nullptr, nullptr, 0, 1));
+            HIPCHK(mfk::oz_gemm_narrow(s, n, nrhs, w.ld, w.dA, w.S, w.dD, w.ld, nrhs * w.ld, w.planes));
+            HIPCHK(mfk::oz_combine(N, s, n, nrhs, U, w.planes, w.eA, w.eD, R));
             clk.mark(ST_RESIDUAL);
         } else {
         // precision of A*D: |D| / |X| = 2^-e needs about (53 N - e) / 52 limbs

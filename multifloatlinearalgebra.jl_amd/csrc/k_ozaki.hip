@@ -2,14 +2,17 @@
 //
 // A Float64xN operand row (or column) is scaled by a power of two 2^e with
 // |value| < 2^(e-2) over the row, converted exactly (up to truncation below
-// 2^(e - 7S)) to a two's complement fixed-point integer Z of 7S bits, and
-// split into S balanced base-128 digits d_s in [-64, 63] (most significant
-// first):   value ~ 2^(e - 7S) * Z,   Z = sum_s d_s 128^(S-1-s).
+// 2^(e - BS)) to a two's complement fixed-point integer Z of BS bits, and
+// split into S balanced digits d_s of B bits in [-2^(B-1), 2^(B-1) - 1] (most
+// significant first):   value ~ 2^(e - BS) * Z,   Z = sum_s d_s 2^(B(S-1-s)).
 // Then
-//   sum_k A(i,k) B(k,j) = sum_{s,t} 2^(ea_i + eb_j - 7(s+t+2)) C_{s,t}(i,j),
+//   sum_k A(i,k) B(k,j) = sum_{s,t} 2^(ea_i + eb_j - B(s+t+2)) C_{s,t}(i,j),
 //   C_{s,t}(i,j) = sum_k dA_s(i,k) dB_t(j,k)          (exact int32)
-// Digit products are at most 2^12 in magnitude, so a group of P pairs over K
-// terms stays below 2^31 while P*K <= 2^18.5 (K <= 8192 with P <= 34).
+// Digit products are at most 2^(2B-2) in magnitude, so a group of P pairs over
+// K terms stays below 2^31 for B = 7 up to K = 8192 (P <= 34), for B = 8 up to
+// K = 4096 (P <= 30). Eight bits need a fifth fewer digit pairs (x4: 30 digits
+// of 8 bits hold 240 bits, 34 of 7 hold 238), so gemm! takes them up to K =
+// 4096; the refinement's A * D keeps 7.
 //
 //  * k_oz_exp_part / k_oz_exp_finish: e_i = ilogb(max_k |hi(X(i,k))|) + 3
 //    (chunked max, fixed order), or a sentinel for all-zero rows.
@@ -19,15 +22,14 @@
 //  * k_oz_round_fp64: a binary64 correction rounded to 7T-bit fixed point per
 //    column (the rounded value is written back, so the caller uses exactly
 //    the value whose digits are multiplied) and split into T digits.
-//  * k_oz_gemm: for every u in [0, U], C_u(i,j) = sum_{s+t=u} sum_k dA_s dB_t
-//    as int32 planes; 128 x 128 (or 128 x 64 for narrow outputs) tile per
-//    256-thread workgroup, each wave a 4 x 4 (4 x 2) block of 16 x 16 MFMA
-//    tiles, 128-byte k-stages prefetched into registers and staged through
-//    padded LDS rows; grid z = u.
-//  * k_oz_combine<N>: acc(i,j) = sum_u C_u(i,j) 2^(ea_i + eb_j - 7(u+2)) in
-//    Float64xN arithmetic, u ascending, then C = alpha*acc + beta*C (or
-//    R = R - acc for a residual update).
+//  * k_oz_gemm: C = alpha*A*B + beta*C; every wave keeps the sums C_u of all
+//    u in [0, S] of one 16 x 16 block in registers and recombines them itself.
+//  * k_oz_gemm_narrow / k_oz_combine<N>: the refinement's A * D as int32
+//    planes C_u, then R = R - acc.
+//  Recombination: acc(i,j) = sum_u C_u(i,j) 2^(ea_i + eb_j - 7(u+2)) in
+//    Float64xN arithmetic, u ascending, four sums at a time (exact in 53 bits).
 #include <climits>
+#include <type_traits>
 #include "mf_common.hpp"
 #include "k_ozaki.hpp"
 
@@ -103,60 +105,46 @@ __device__ __forceinline__ void acc_add_shifted(Acc256 &a, uint64_t mag, int sh,
     }
 }
 
-// digits of a 7S-bit value held in a 256-bit accumulator: balanced base 128,
-// least significant first into d[S-1], ..., most significant into d[0]
-__device__ __forceinline__ void acc_digits(const Acc256 &a, int S, int8_t *d, int64_t stride) {
-    int carry = 0;
-    for (int q = 0; q < S; ++q) {
-        const int bit = 7 * q;
-        const int wq = bit >> 6, bq = bit & 63;
-        uint64_t chunk = a.w[wq] >> bq;
-        if (bq > 57 && wq + 1 < 4) chunk |= a.w[wq + 1] << (64 - bq);
-        int b = (int)(chunk & 127) + carry;
-        int dig;
-        if (b >= 64) { dig = b - 128; carry = 1; } else { dig = b; carry = 0; }
-        d[(int64_t)(S - 1 - q) * stride] = (int8_t)dig;
-    }
-}
-
-// acc_digits with the digit count a compile-time constant: every word index
-// and shift is static (the runtime form selects among the four words per
-// digit).
-template <int S>
-__device__ __forceinline__ void acc_digits_t(const Acc256 &a, int8_t *d, int64_t stride) {
+// The S digits of B bits of a value held in a 256-bit accumulator, balanced,
+// least significant first into d[S-1], ..., most significant into d[0]. S
+// and B are constants, so every word index and shift is static.
+template <int S, int B>
+__device__ __forceinline__ void acc_digits(const Acc256 &a, int8_t *d, int64_t stride) {
+    static_assert(B * S <= 250, "the accumulator holds the digits");
+    constexpr int BASE = 1 << B;
     int carry = 0;
 #pragma unroll
     for (int q = 0; q < S; ++q) {
-        const int bit = 7 * q;
+        const int bit = B * q;
         const int wq = bit >> 6, bq = bit & 63;
         uint64_t chunk = a.w[wq] >> bq;
-        if (bq > 57 && wq + 1 < 4) chunk |= a.w[wq + 1] << (64 - bq);
-        int b = (int)(chunk & 127) + carry;
+        if (bq > 64 - B && wq + 1 < 4) chunk |= a.w[wq + 1] << (64 - bq);
+        int b = (int)(chunk & (BASE - 1)) + carry;
         int dig;
-        if (b >= 64) { dig = b - 128; carry = 1; } else { dig = b; carry = 0; }
+        if (b >= BASE / 2) { dig = b - BASE; carry = 1; } else { dig = b; carry = 0; }
         d[(int64_t)(S - 1 - q) * stride] = (int8_t)dig;
     }
 }
 
-// Byte offset of digit (i, k) inside one digit plane. Row layout: i * ld +
-// k. Fragment layout (FRAG): 16-row blocks, each a sequence of 64-deep k
-// steps of 1 KB laid out exactly as the lanes of a wave read one MFMA
-// 16x16x64 fragment (lane l = 16 * (k % 64 / 16) + i % 16 takes 16
-// consecutive k), so a wave's fragment load is one contiguous 1 KB block.
-template <bool FRAG>
-__device__ __forceinline__ int64_t oz_off(int64_t i, int64_t k, int64_t ld) {
-    if (!FRAG) return i * ld + k;
-    return ((i >> 4) * (ld >> 6) + (k >> 6)) * 1024 + ((((k & 63) >> 4) << 4) + (i & 15)) * 16 + (k & 15);
+// Digits of X(i, k) as MFMA fragments: 16-row blocks, each a sequence of
+// 64-deep k steps, each the S digits' 16x16x64 fragments of 1 KB, laid out
+// exactly as the lanes of a wave read one (lane l = 16 * (k % 64 / 16) + i %
+// 16 takes 16 consecutive k). A wave's load is one contiguous 1 KB and the
+// digits it multiplies together are adjacent. Offset of digit 0:
+constexpr int64_t OZ_FRAG = 1024;
+__device__ __forceinline__ int64_t oz_off(int64_t i, int64_t k, int64_t ld, int S) {
+    return ((i >> 4) * (ld >> 6) + (k >> 6)) * S * OZ_FRAG + ((((k & 63) >> 4) << 4) + (i & 15)) * 16 + (k & 15);
 }
 
-// dig[s * plane + oz_off(i, k)] for X(i, k), s = 0..S-1; the padding
-// columns k in [K, ld) get zero digits.
-template <int N, bool FRAG, int SC>
-__global__ void k_oz_split(int64_t m, int64_t K, DV X, int uplo, const int *e, int S, int8_t *dig, int64_t ld, int64_t plane) {
+// digits s = 0..S-1 of X(i, k); the padding columns k in [K, ld) get zero
+// digits, the rows that fill the last block of 16 are left as they are (they
+// reach only outputs that are not stored).
+template <int N, int S, int B>
+__global__ void k_oz_split(int64_t m, int64_t K, DV X, int uplo, const int *e, int8_t *dig, int64_t ld) {
     const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (idx >= m * ld) return;
     const int64_t k = idx % ld, i = idx / ld;        // k fastest: coalesced digit stores
-    int8_t *d = dig + oz_off<FRAG>(i, k, ld);
+    int8_t *d = dig + oz_off(i, k, ld, S);
     const int ei = e[i];
     Acc256 a{{0, 0, 0, 0}};
     if (ei != OZ_ZERO_ROW && k < K) {
@@ -168,11 +156,10 @@ __global__ void k_oz_split(int64_t m, int64_t K, DV X, int uplo, const int *e, i
             int ex;
             const double f = frexp(fabs(x), &ex);                 // |x| = f 2^ex, f in [0.5, 1)
             const uint64_t mag = (uint64_t)ldexp(f, 53);            // 53-bit integer mantissa
-            acc_add_shifted(a, mag, ex - 53 + 7 * (SC > 0 ? SC : S) - ei, x < 0.0);
+            acc_add_shifted(a, mag, ex - 53 + B * S - ei, x < 0.0);
         }
     }
-    if constexpr (SC > 0) acc_digits_t<SC>(a, d, plane);
-    else acc_digits(a, S, d, plane);
+    acc_digits<S, B>(a, d, OZ_FRAG);
 }
 
 // binary64 correction D(k, j) (k in [0, K), column j): per-column exponent
@@ -208,93 +195,145 @@ __global__ void k_oz_round_fp64(int64_t K, int64_t ncols, DV D, const int *e, in
 // ----------------------------------------------------------- INT8 GEMM
 typedef int v4i __attribute__((ext_vector_type(4)));
 
-// out[u * m * n + j * m + i] = sum_{s + t = u, s < SA, t < SB} sum_k dA_s(i,k) dB_t(j,k)
-// K is the padded length of the digit rows (a multiple of OZ_KS); padding
-// digits are zero. Workgroup tile (32 WM) x (32 WN) from 2 x 2 waves of
-// WM x WN MFMA 16x16x64 blocks; every (plane s, 128-byte k-stage) is one
-// stage of the loop, with the next stage prefetched into registers while
-// the current one is multiplied from LDS. LDS rows are padded to 144 bytes
-// so the 16 rows a lane group reads fall on distinct banks.
-constexpr int OZ_KS = 128, OZ_LDW = 144;
 constexpr int OZ_NARROW_TB = 6;   // B digits of the narrow kernel (binary64 corrections)
 
-template <int WM, int WN>
-__global__ __launch_bounds__(256) void k_oz_gemm(int64_t m, int64_t n, int64_t K, const int8_t *dA, int64_t lda, int64_t planeA,
-                                                 int SA, const int8_t *dB, int64_t ldb, int64_t planeB, int SB, int32_t *out,
-                                                 int tiles_m) {
-    constexpr int TM = 32 * WM, TN = 32 * WN;
-    constexpr int CA = TM * (OZ_KS / 16) / 256, CB = TN * (OZ_KS / 16) / 256;   // 16-byte chunks per thread
-    __shared__ __align__(16) int8_t As[TM * OZ_LDW];
-    __shared__ __align__(16) int8_t Bs[TN * OZ_LDW];
-    const int t = threadIdx.x, lane = t & 63, w = t >> 6;
-    const int wy = w & 1, wx = w >> 1;
-    const int64_t i0 = (int64_t)(blockIdx.x % tiles_m) * TM, j0 = (int64_t)(blockIdx.x / tiles_m) * TN;
-    const int u = (int)blockIdx.z;
-    const int slo = u - (SB - 1) > 0 ? u - (SB - 1) : 0, shi = u < SA - 1 ? u : SA - 1;
-    const int64_t kst = K / OZ_KS;
-    const int64_t stages = (int64_t)(shi - slo + 1) * kst;
-    v4i acc[WM][WN];
+// Sums of U + 1 digit planes (B-bit digits) to Float64xN: c(u) weighs
+// 2^(base - B(u + 2)). As many consecutive planes as stay below 2^53 together
+// (|c| < 2^31) are one integer, so they enter the Float64xN sum exactly and
+// as one binary64 value.
+template <int N, int B, typename C> __device__ __forceinline__ mf::V<N> oz_sum(int U, int base, const C &c) {
+    constexpr int G = 1 + 21 / B;
+    mf::V<N> acc = mf::zero<N>();
+    int u = 0;
 #pragma unroll
-    for (int a = 0; a < WM; ++a)
+    for (; u + G - 1 <= U; u += G) {
+        int64_t v = c(u);
 #pragma unroll
-        for (int b = 0; b < WN; ++b) acc[a][b] = v4i{0, 0, 0, 0};
-    v4i ra[CA], rb[CB];
-    auto fetch = [&](int64_t g) {
-        const int sp = slo + (int)(g / kst);
-        const int64_t k0 = (g % kst) * OZ_KS;
-        const int8_t *pa = dA + (int64_t)sp * planeA + k0, *pb = dB + (int64_t)(u - sp) * planeB + k0;
-#pragma unroll
-        for (int q = 0; q < CA; ++q) {
-            const int c = t + 256 * q, r = c / (OZ_KS / 16), col = (c % (OZ_KS / 16)) * 16;
-            ra[q] = (i0 + r < m) ? *(const v4i *)(pa + (i0 + r) * lda + col) : v4i{0, 0, 0, 0};
-        }
-#pragma unroll
-        for (int q = 0; q < CB; ++q) {
-            const int c = t + 256 * q, r = c / (OZ_KS / 16), col = (c % (OZ_KS / 16)) * 16;
-            rb[q] = (j0 + r < n) ? *(const v4i *)(pb + (j0 + r) * ldb + col) : v4i{0, 0, 0, 0};
-        }
-    };
-    if (stages > 0) fetch(0);
-    for (int64_t g = 0; g < stages; ++g) {
-#pragma unroll
-        for (int q = 0; q < CA; ++q) {
-            const int c = t + 256 * q, r = c / (OZ_KS / 16), col = (c % (OZ_KS / 16)) * 16;
-            *(v4i *)(As + r * OZ_LDW + col) = ra[q];
-        }
-#pragma unroll
-        for (int q = 0; q < CB; ++q) {
-            const int c = t + 256 * q, r = c / (OZ_KS / 16), col = (c % (OZ_KS / 16)) * 16;
-            *(v4i *)(Bs + r * OZ_LDW + col) = rb[q];
-        }
-        __syncthreads();
-        if (g + 1 < stages) fetch(g + 1);
-#pragma unroll
-        for (int ks = 0; ks < OZ_KS / 64; ++ks) {
-            v4i fa[WM], fb[WN];
-#pragma unroll
-            for (int a = 0; a < WM; ++a) fa[a] = *(const v4i *)(As + (wy * 16 * WM + a * 16 + (lane & 15)) * OZ_LDW + ks * 64 + (lane >> 4) * 16);
-#pragma unroll
-            for (int b = 0; b < WN; ++b) fb[b] = *(const v4i *)(Bs + (wx * 16 * WN + b * 16 + (lane & 15)) * OZ_LDW + ks * 64 + (lane >> 4) * 16);
-#pragma unroll
-            for (int a = 0; a < WM; ++a)
-#pragma unroll
-                for (int b = 0; b < WN; ++b) acc[a][b] = __builtin_amdgcn_mfma_i32_16x16x64_i8(fb[b], fa[a], acc[a][b], 0, 0, 0);
-        }
-        __syncthreads();
+        for (int g = 1; g < G; ++g) v = (v << B) + c(u + g);
+        acc = mf::add(acc, mf::from<N>(ldexp((double)v, base - B * (u + G + 1))));
     }
-    // with the B fragment first, item v of lane l holds row (lane % 16) and
-    // column 4 (lane / 16) + v of the 16 x 16 block: coalesced column stores
-    int32_t *o = out + (int64_t)u * m * n;
 #pragma unroll
-    for (int a = 0; a < WM; ++a)
+    for (; u <= U; ++u) acc = mf::add(acc, mf::from<N>(ldexp((double)c(u), base - B * (u + 2))));
+    return acc;
+}
+
+// C = alpha*A*B + beta*C from the digits of A's rows and B's columns (both in
+// the fragment layout, S digits each, `steps` k steps). A wave computes WN
+// 16 x 16 blocks side by side with the sums C_u of all u <= S in registers
+// (S + 1 fragments of 4 each: 124 for S = 30) beside A's S fragments of a k
+// step: the 60 KB of digits of a step feed (S + 1)(S + 2) / 2 - 2 = 494 MFMAs
+// (7900 cycles), so the operands stream from L2 at 8 bytes a cycle and wave
+// (6 with WN = 2) and need neither LDS nor barriers. (One plane u per pass over
+// 128 x 128 LDS tiles read 128 bytes of LDS a cycle, its peak, for MFMAs that
+// ran at 28 % of theirs, and wrote the planes out for another kernel to sum:
+// whole gemm! x4 2048^3 7.82 ms, x3 4.97, x2 2.68; so 3.84, 2.42, 1.55, the
+// x4 kernel at 2400 TOP/s where a large bf16 matrix product reaches 54 % of
+// its nominal rate on the same card and this 48 % of 5.0 POP/s.)
+// B's fragments run OZ_AHEAD ahead; a fragment of A is replaced by the next
+// step's after its last MFMA, the first OZ_EARLY (whose last MFMAs end the
+// step) are fetched into registers of their own.
+// KS = 1: the four waves of a workgroup take a tile of 2 x 2 wave blocks.
+// KS = 4: they share one and take every fourth k step each, add their sums
+// (integers: any order) through LDS and finish every fourth column each.
+template <int N, int B, int S, int KS, int WN, int OZ_AHEAD, int OZ_EARLY>
+__global__ __launch_bounds__(256, 1) void k_oz_gemm(int64_t m, int64_t n, int steps, const int8_t *dA, const int8_t *dB, const int *ea,
+                                                    const int *eb, DV C, mfk::S<N> alpha, mfk::S<N> beta, int beta_zero, int tiles_m, int tiles_n,
+                                                    int per_xcd) {
+    constexpr int U = S;
+    static_assert(2 * OZ_EARLY <= S - 1 && OZ_AHEAD < S, "the prefetches stay within one step");
+    constexpr int64_t STEP = S * OZ_FRAG;
+    const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+    // workgroup b runs on XCD b % 8: each XCD takes a contiguous run of tiles,
+    // enumerated in bands of 8 tile rows, so the ~32 tiles it holds at once
+    // share rows and columns in its L2
+    const int64_t tile = (int64_t)(blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
+    if (tile >= (int64_t)tiles_m * tiles_n) return;
+    const int64_t band = tile / (8 * tiles_n), in = tile - band * 8 * tiles_n;
+    const int64_t high = tiles_m - band * 8 < 8 ? tiles_m - band * 8 : 8;
+    const int64_t bi = band * 8 + in % high, bj = in / high;
+    const int64_t ib = KS == 1 ? bi * 2 + (w & 1) : bi, jb = (KS == 1 ? bj * 2 + (w >> 1) : bj) * WN;   // 16-row / 16-column blocks
+    if (ib * 16 >= m || jb * 16 >= n) return;            // KS == 1 only: no barrier follows
+    v4i acc[WN][U + 1];
 #pragma unroll
-        for (int b = 0; b < WN; ++b)
+    for (int h = 0; h < WN; ++h)
+#pragma unroll
+        for (int u = 0; u <= U; ++u) acc[h][u] = v4i{0, 0, 0, 0};
+    const int first = KS == 1 ? 0 : w;
+    if (first < steps) {
+        static_assert(WN <= 2, "one block may be missing at the right edge");
+        const int64_t bcol = (jb + 1) * 16 < n ? steps * STEP : 0;   // to the second column block, if B has one
+        const int8_t *pa = dA + (ib * steps + first) * STEP + lane * 16, *pb = dB + (jb * steps + first) * STEP + lane * 16;
+        auto frag = [](const int8_t *p, int s) { return *(const v4i *)(p + s * OZ_FRAG); };
+        v4i fa[S], fb[WN][OZ_AHEAD], early[OZ_EARLY];
+#pragma unroll
+        for (int s = S - 1; s >= 0; --s) fa[s] = frag(pa, s);
+#pragma unroll
+        for (int q = 0; q < OZ_AHEAD; ++q)
+#pragma unroll
+            for (int h = 0; h < WN; ++h) fb[h][q] = frag(pb + h * bcol, q);
+        for (int ks = first; ks < steps; ks += KS) {
+            // the last step fetches its own fragments again instead of a step past the end
+            const int8_t *na = ks + KS < steps ? pa + KS * STEP : pa, *nb = ks + KS < steps ? pb + KS * STEP : pb;
+#pragma unroll
+            for (int q = 0; q < S; ++q) {
+                v4i b[WN];
+#pragma unroll
+                for (int h = 0; h < WN; ++h) {
+                    b[h] = fb[h][0];
+#pragma unroll
+                    for (int x = 0; x + 1 < OZ_AHEAD; ++x) fb[h][x] = fb[h][x + 1];
+                    fb[h][OZ_AHEAD - 1] = q + OZ_AHEAD < S ? frag(pb + h * bcol, q + OZ_AHEAD) : frag(nb + h * bcol, q + OZ_AHEAD - S);
+                }
+                if (q >= S - 1 - 2 * OZ_EARLY && q < S - 1 - OZ_EARLY) early[q - (S - 1 - 2 * OZ_EARLY)] = frag(na, q - (S - 1 - 2 * OZ_EARLY));
+#pragma unroll
+                for (int x = S - 1; x >= 0; --x)
+#pragma unroll
+                    for (int h = 0; h < WN; ++h)
+                        if (x + q <= U) acc[h][x + q] = __builtin_amdgcn_mfma_i32_16x16x64_i8(b[h], fa[x], acc[h][x + q], 0, 0, 0);
+                if (q >= 1 && U - q >= OZ_EARLY) fa[U - q] = frag(na, U - q);
+            }
+#pragma unroll
+            for (int x = 0; x < OZ_EARLY; ++x) fa[x] = early[x];
+            pa = na;
+            pb = nb;
+        }
+    }
+    const mf::V<N> al = sv(alpha), be = sv(beta);
+    // item v of lane l: row l % 16, column 4 (l / 16) + v of the block
+    const int64_t i = ib * 16 + (lane & 15);
+    auto finish = [&](int h, int v, auto sums) {
+        const int64_t j = (jb + h) * 16 + 4 * (lane >> 4) + v;
+        if (i >= m || j >= n) return;
+        const int xa = ea[i], xb = eb[j];
+        const mf::V<N> p = xa == OZ_ZERO_ROW || xb == OZ_ZERO_ROW ? mf::zero<N>() : oz_sum<N, B>(U, xa + xb, sums);
+        stv<N>(C, i, j, beta_zero ? mf::mul(al, p) : mf::add(mf::mul(al, p), mf::mul(be, ld<N>(C, i, j))));
+    };
+    if constexpr (KS == 1) {
+#pragma unroll
+        for (int h = 0; h < WN; ++h)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) finish(h, v, [&](int u) { return acc[h][u][v]; });
+    } else {
+        __shared__ int32_t part[3][U + 1][64];
+#pragma unroll
+        for (int h = 0; h < WN; ++h) {
+            int32_t mine[U + 1];
 #pragma unroll
             for (int v = 0; v < 4; ++v) {
-                const int64_t i = i0 + wy * 16 * WM + a * 16 + (lane & 15);
-                const int64_t j = j0 + wx * 16 * WN + b * 16 + 4 * (lane >> 4) + v;
-                if (i < m && j < n) o[j * m + i] = acc[a][b][v];
+                if (w != v) {
+#pragma unroll
+                    for (int u = 0; u <= U; ++u) part[w < v ? w : w - 1][u][lane] = acc[h][u][v];
+                }
+                __syncthreads();
+                if (w == v) {
+#pragma unroll
+                    for (int u = 0; u <= U; ++u) mine[u] = acc[h][u][v] + part[0][u][lane] + part[1][u][lane] + part[2][u][lane];
+                }
+                __syncthreads();
             }
+            finish(h, w, [&](int u) { return mine[u]; });
+        }
+    }
 }
 
 // Narrow products (the refinement's A * D: few columns, TB = 6 digits of a
@@ -307,15 +346,14 @@ __global__ __launch_bounds__(256) void k_oz_gemm(int64_t m, int64_t n, int64_t K
 // s into the planes s .. s + TB - 1. A workgroup is 16 rows x 64 columns
 // (four waves side by side); grid.y runs over 64-column groups.
 template <int SA, int TB>
-__global__ __launch_bounds__(256) void k_oz_gemm_narrow(int64_t m, int64_t n, int64_t K, const int8_t *dA, int64_t planeA,
-                                                        const int8_t *dB, int64_t ldb, int64_t planeB, int32_t *out) {
+__global__ __launch_bounds__(256) void k_oz_gemm_narrow(int64_t m, int64_t n, int64_t K, const int8_t *dA, const int8_t *dB, int64_t ldb, int64_t planeB, int32_t *out) {
     constexpr int NP = SA + TB - 1;
     const int t = threadIdx.x, lane = t & 63, w = t >> 6;
     const int64_t i0 = (int64_t)blockIdx.x * 16, j0 = (int64_t)blockIdx.y * 64 + (int64_t)w * 16;
     const int64_t ia = i0 + (lane & 15), jb = j0 + (lane & 15);
     const bool rowok = ia < m, colok = jb < n;
     // the fragment layout pads the rows to 16, so every A load is in bounds
-    const int8_t *pa = dA + (int64_t)blockIdx.x * (K >> 6) * 1024 + lane * 16;
+    const int8_t *pa = dA + (int64_t)blockIdx.x * (K >> 6) * SA * OZ_FRAG + lane * 16;
     const int8_t *pb = dB + (colok ? jb : 0) * ldb + (lane >> 4) * 16;
     v4i acc[NP];
 #pragma unroll
@@ -324,13 +362,13 @@ __global__ __launch_bounds__(256) void k_oz_gemm_narrow(int64_t m, int64_t n, in
     // the next step right after its MFMAs are issued
     v4i fa[SA], fb[TB];
 #pragma unroll
-    for (int s = 0; s < SA; ++s) fa[s] = *(const v4i *)(pa + s * planeA);
+    for (int s = 0; s < SA; ++s) fa[s] = *(const v4i *)(pa + s * OZ_FRAG);
 #pragma unroll
     for (int q = 0; q < TB; ++q) fb[q] = *(const v4i *)(pb + q * planeB);
     const v4i zero{0, 0, 0, 0};
     for (int64_t k0 = 0; k0 < K; k0 += 64) {
         const bool more = k0 + 64 < K;
-        const int8_t *pn = pa + ((k0 + 64) >> 6) * 1024;
+        const int8_t *pn = pa + ((k0 + 64) >> 6) * SA * OZ_FRAG;
         v4i gb[TB];
 #pragma unroll
         for (int q = 0; q < TB; ++q) gb[q] = colok ? fb[q] : zero;
@@ -343,7 +381,7 @@ __global__ __launch_bounds__(256) void k_oz_gemm_narrow(int64_t m, int64_t n, in
             const v4i a = fa[s];
 #pragma unroll
             for (int q = 0; q < TB; ++q) acc[s + q] = __builtin_amdgcn_mfma_i32_16x16x64_i8(gb[q], a, acc[s + q], 0, 0, 0);
-            if (more) fa[s] = *(const v4i *)(pn + s * planeA);
+            if (more) fa[s] = *(const v4i *)(pn + s * OZ_FRAG);
         }
     }
     // item v of lane l: row (lane % 16), column 4 (lane / 16) + v of the block
@@ -359,11 +397,9 @@ __global__ __launch_bounds__(256) void k_oz_gemm_narrow(int64_t m, int64_t n, in
 }
 
 // -------------------------------------------------------------- combine
-// acc = sum_u C_u 2^(ea_i + eb_j - 7(u + 2)), u ascending, in N limbs; then
-// mode 0: C = alpha*acc (beta == 0) or alpha*acc + beta*C; mode 1: C = C - acc.
+// C -= sum_u C_u 2^(ea_i + eb_j - 7(u + 2)), u ascending, in N limbs
 template <int N>
-__global__ void k_oz_combine(int64_t m, int64_t n, int U, const int32_t *planes, const int *ea, const int *eb, DV C, S<N> alpha,
-                             S<N> beta, int beta_zero, int mode) {
+__global__ void k_oz_combine(int64_t m, int64_t n, int U, const int32_t *planes, const int *ea, const int *eb, DV C) {
     const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (idx >= m * n) return;
     const int64_t i = idx % m, j = idx / m;
@@ -375,11 +411,7 @@ __global__ void k_oz_combine(int64_t m, int64_t n, int U, const int32_t *planes,
             if (c != 0) acc = mf::add(acc, mf::from<N>(ldexp((double)c, base - 7 * (u + 2))));
         }
     }
-    mf::V<N> r;
-    if (mode == 1) r = mf::sub(ld<N>(C, i, j), acc);
-    else if (beta_zero) r = mf::mul(sv(alpha), acc);
-    else r = mf::add(mf::mul(sv(alpha), acc), mf::mul(sv(beta), ld<N>(C, i, j)));
-    stv<N>(C, i, j, r);
+    stv<N>(C, i, j, mf::sub(ld<N>(C, i, j), acc));
 }
 
 // ---------------------------------------------------------- launchers
@@ -406,39 +438,46 @@ hipError_t oz_exponents(hipStream_t s, int64_t m, int64_t K, const DV &X, int up
     return hipGetLastError();
 }
 
-hipError_t oz_split(int N, hipStream_t s, int64_t m, int64_t K, const DV &X, int uplo, const int *e, int S, int8_t *dig, int64_t ld,
-                    int64_t plane, bool frag) {
+int64_t oz_bytes(int64_t m, int64_t ld, int S) { return cdiv(m, 16) * 16 * ld * S; }
+
+// gemm!'s digits: 8 bits while the int32 sums hold them
+int oz_gemm_digits(int N, int64_t K) {
+    if (K > 4096) return oz_digits(N);
+    return N >= 4 ? 30 : (N == 3 ? 24 : (N == 2 ? 17 : 10));
+}
+
+hipError_t oz_split(int N, hipStream_t s, int64_t m, int64_t K, const DV &X, int uplo, const int *e, int S, int8_t *dig, int64_t ld) {
     if (m * ld == 0) return hipSuccess;
-    if (S < 1 || 7 * S > 250 || ld % 64 != 0 || ld < K) return hipErrorInvalidValue;
-    if (frag && plane < cdiv(m, 16) * 16 * ld) return hipErrorInvalidValue;
+    if (ld % 64 != 0 || ld < K) return hipErrorInvalidValue;
     const dim3 grid((unsigned)cdiv(m * ld, 256));
-#define OZ_SPLIT(F, SCV) OZ_DISPATCH(N, hipLaunchKernelGGL((k_oz_split<NN, F, SCV>), grid, dim3(256), 0, s, m, K, X, uplo, e, S, dig, ld, plane))
-#define OZ_SPLIT_S(F)                                            \
-    switch (S) {                                                 \
-        case 11: OZ_SPLIT(F, 11); break;                         \
-        case 19: OZ_SPLIT(F, 19); break;                         \
-        case 27: OZ_SPLIT(F, 27); break;                         \
-        case 34: OZ_SPLIT(F, 34); break;                         \
-        default: OZ_SPLIT(F, 0); break;                          \
+#define OZ_SPLIT(SC, B) OZ_DISPATCH(N, hipLaunchKernelGGL((k_oz_split<NN, SC, B>), grid, dim3(256), 0, s, m, K, X, uplo, e, dig, ld))
+    switch (S) {   // the digit counts of oz_digits and oz_gemm_digits
+        case 11: OZ_SPLIT(11, 7); break;
+        case 19: OZ_SPLIT(19, 7); break;
+        case 27: OZ_SPLIT(27, 7); break;
+        case 34: OZ_SPLIT(34, 7); break;
+        case 10: OZ_SPLIT(10, 8); break;
+        case 17: OZ_SPLIT(17, 8); break;
+        case 24: OZ_SPLIT(24, 8); break;
+        case 30: OZ_SPLIT(30, 8); break;
+        default: return hipErrorInvalidValue;
     }
-    if (frag) { OZ_SPLIT_S(true) } else { OZ_SPLIT_S(false) }
-#undef OZ_SPLIT_S
 #undef OZ_SPLIT
     return hipGetLastError();
 }
 
 int oz_narrow_digits() { return OZ_NARROW_TB; }
 
-hipError_t oz_gemm_narrow(hipStream_t s, int64_t m, int64_t n, int64_t K, const int8_t *dA, int64_t planeA, int SA, const int8_t *dB,
-                          int64_t ldb, int64_t planeB, int32_t *out) {
+hipError_t oz_gemm_narrow(hipStream_t s, int64_t m, int64_t n, int64_t K, const int8_t *dA, int SA, const int8_t *dB, int64_t ldb,
+                          int64_t planeB, int32_t *out) {
     if (m == 0 || n == 0) return hipSuccess;
-    if (K > 8192 || K % OZ_KS != 0 || ldb % 16 != 0 || planeA < cdiv(m, 16) * 16 * K) return hipErrorInvalidValue;
+    if (K > 8192 || K % 64 != 0 || ldb % 16 != 0) return hipErrorInvalidValue;
     const dim3 grid((unsigned)cdiv(m, 16), (unsigned)cdiv(n, 64)), block(256);
     switch (SA) {   // the digit counts of oz_digits(N)
-        case 34: hipLaunchKernelGGL((k_oz_gemm_narrow<34, OZ_NARROW_TB>), grid, block, 0, s, m, n, K, dA, planeA, dB, ldb, planeB, out); break;
-        case 27: hipLaunchKernelGGL((k_oz_gemm_narrow<27, OZ_NARROW_TB>), grid, block, 0, s, m, n, K, dA, planeA, dB, ldb, planeB, out); break;
-        case 19: hipLaunchKernelGGL((k_oz_gemm_narrow<19, OZ_NARROW_TB>), grid, block, 0, s, m, n, K, dA, planeA, dB, ldb, planeB, out); break;
-        case 11: hipLaunchKernelGGL((k_oz_gemm_narrow<11, OZ_NARROW_TB>), grid, block, 0, s, m, n, K, dA, planeA, dB, ldb, planeB, out); break;
+        case 34: hipLaunchKernelGGL((k_oz_gemm_narrow<34, OZ_NARROW_TB>), grid, block, 0, s, m, n, K, dA, dB, ldb, planeB, out); break;
+        case 27: hipLaunchKernelGGL((k_oz_gemm_narrow<27, OZ_NARROW_TB>), grid, block, 0, s, m, n, K, dA, dB, ldb, planeB, out); break;
+        case 19: hipLaunchKernelGGL((k_oz_gemm_narrow<19, OZ_NARROW_TB>), grid, block, 0, s, m, n, K, dA, dB, ldb, planeB, out); break;
+        case 11: hipLaunchKernelGGL((k_oz_gemm_narrow<11, OZ_NARROW_TB>), grid, block, 0, s, m, n, K, dA, dB, ldb, planeB, out); break;
         default: return hipErrorInvalidValue;
     }
     return hipGetLastError();
@@ -452,31 +491,54 @@ hipError_t oz_round_fp64(hipStream_t s, int64_t K, int64_t ncols, const DV &D, c
     return hipGetLastError();
 }
 
-hipError_t oz_gemm(hipStream_t s, int64_t m, int64_t n, int64_t K, const int8_t *dA, int64_t lda, int64_t planeA, int SA,
-                   const int8_t *dB, int64_t ldb, int64_t planeB, int SB, int U, int32_t *out) {
-    if (m == 0 || n == 0) return hipSuccess;
-    // int32 headroom: pairs * K * 2^12 < 2^31
-    if (K > 8192 || K % OZ_KS != 0 || lda % 16 != 0 || ldb % 16 != 0 || (SA < SB ? SA : SB) > 34 || U > SA + SB - 2)
-        return hipErrorInvalidValue;
-    if (n <= 64) {
-        const int tiles_m = (int)cdiv(m, 128);
-        const dim3 grid((unsigned)(tiles_m * cdiv(n, 64)), 1, (unsigned)(U + 1));
-        hipLaunchKernelGGL((k_oz_gemm<4, 2>), grid, dim3(256), 0, s, m, n, K, dA, lda, planeA, SA, dB, ldb, planeB, SB, out, tiles_m);
-    } else {
-        const int tiles_m = (int)cdiv(m, 128);
-        const dim3 grid((unsigned)(tiles_m * cdiv(n, 128)), 1, (unsigned)(U + 1));
-        hipLaunchKernelGGL((k_oz_gemm<4, 4>), grid, dim3(256), 0, s, m, n, K, dA, lda, planeA, SA, dB, ldb, planeB, SB, out, tiles_m);
-    }
+// Workgroup shapes, by the number of 16 x 16 blocks (the gemm kernel alone,
+// 512^3 / 1024^3 / 2048^3 / 4096^3): four limbs share two blocks side by side
+// from 4096 blocks on (0.086 / 0.495 / 3.54 / 28.3 ms), give each wave a block
+// from 1024 on, one block for each SIMD (0.072 / 0.473 / 4.02 / 31.0), and
+// share one block below (0.097 / 0.601 / 4.65 / 37.9, but four times the
+// workgroups). Fewer limbs share one block at every size (x3 0.049 / 0.284 /
+// 2.08 / 17.8 against 0.055 / 0.334 / 2.21 / 19.6 for two, x2 0.029 / 0.177 /
+// 1.34 / 11.5 against 0.033 / 0.224 / 1.60 / 15.1).
+template <int N, int B, int S, int KS, int WN, int AHEAD, int EARLY>
+static hipError_t oz_launch(hipStream_t s, int64_t m, int64_t n, int64_t K, const int8_t *dA, const int8_t *dB, const int *ea, const int *eb,
+                            const DV &C, const double *alpha, const double *beta, int beta_zero) {
+    const int64_t bm = cdiv(m, 16), bn = cdiv(n, 16 * WN);
+    const int64_t tm = KS == 1 ? cdiv(bm, 2) : bm, tn = KS == 1 ? cdiv(bn, 2) : bn, per = cdiv(tm * tn, 8);
+    if (per * 8 > INT32_MAX) return hipErrorInvalidValue;
+    hipLaunchKernelGGL((k_oz_gemm<N, B, S, KS, WN, AHEAD, EARLY>), dim3((unsigned)(per * 8)), dim3(256), 0, s, m, n, (int)(K / 64), dA, dB, ea,
+                       eb, C, mk_oz<N>(alpha), mk_oz<N>(beta), beta_zero, (int)tm, (int)tn, (int)per);
     return hipGetLastError();
 }
 
-int oz_row_align() { return OZ_KS; }
+hipError_t oz_gemm(int N, hipStream_t s, int64_t m, int64_t n, int64_t K, int S, const int8_t *dA, const int8_t *dB, const int *ea,
+                   const int *eb, const DV &C, const double *alpha, const double *beta, int beta_zero) {
+    if (m == 0 || n == 0) return hipSuccess;
+    if (K > 8192 || K % 64 != 0 || S != oz_gemm_digits(N, K)) return hipErrorInvalidValue;
+    const int64_t blocks = cdiv(m, 16) * cdiv(n, 16);
+#define OZ_GO(...) return oz_launch<__VA_ARGS__>(s, m, n, K, dA, dB, ea, eb, C, alpha, beta, beta_zero)
+    switch (S) {
+        case 30:
+            if (blocks >= 4096) OZ_GO(4, 8, 30, 4, 2, 3, 6);
+            if (blocks >= 1024) OZ_GO(4, 8, 30, 1, 1, 4, 6);
+            OZ_GO(4, 8, 30, 4, 1, 8, 6);
+        case 24: OZ_GO(3, 8, 24, 4, 1, 8, 6);
+        case 17: OZ_GO(2, 8, 17, 4, 1, 8, 6);
+        case 10: OZ_GO(1, 8, 10, 4, 1, 4, 4);
+        case 34: OZ_GO(4, 7, 34, 4, 1, 8, 6);
+        case 27: OZ_GO(3, 7, 27, 4, 2, 6, 6);   // one block: 8.6 ms for 2000 x 6000 x 1000
+        case 19: OZ_GO(2, 7, 19, 4, 1, 8, 6);
+        case 11: OZ_GO(1, 7, 11, 4, 1, 4, 5);
+    }
+#undef OZ_GO
+    return hipErrorInvalidValue;
+}
+
+int oz_row_align() { return 64; }
 
 hipError_t oz_combine(int N, hipStream_t s, int64_t m, int64_t n, int U, const int32_t *planes, const int *ea, const int *eb,
-                      const DV &C, const double *alpha, const double *beta, int beta_zero, int mode) {
+                      const DV &C) {
     if (m * n == 0) return hipSuccess;
-    OZ_DISPATCH(N, hipLaunchKernelGGL(k_oz_combine<NN>, dim3((unsigned)cdiv(m * n, 256)), dim3(256), 0, s, m, n, U, planes, ea, eb, C,
-                                      mk_oz<NN>(alpha), mk_oz<NN>(beta), beta_zero, mode));
+    OZ_DISPATCH(N, hipLaunchKernelGGL(k_oz_combine<NN>, dim3((unsigned)cdiv(m * n, 256)), dim3(256), 0, s, m, n, U, planes, ea, eb, C));
     return hipGetLastError();
 }
 
