@@ -877,6 +877,37 @@ int mfla_potrf(mfla_handle h, int N, mfla_matrix A, int64_t *info, const mfla_co
         HIPCHK(hipEventRecord(h->ev_join, s));
         HIPCHK(hipStreamWaitEvent(s1, h->ev_join, 0));
     }
+    // Panels of up to 16 columns: one kernel per panel (chol_step: the update
+    // of its columns by the panel before, the panel, the rows below), the
+    // update of the columns beyond the next panel on the second stream.
+    if (block <= 16 && n > 0) {
+        double *diag = (double *)grow_scratch(h, mfk::chol_step_doubles(N, n) * sizeof(double));
+        if (!diag) return fail(MFLA_ERR_HIP, "scratch allocation failed");
+        const hipEvent_t updated[2] = {h->ev_update, h->ev_update2};   // by the panel's parity
+        int64_t p = 0;
+        for (int64_t first = 0; first < n; first += block, ++p) {
+            const int64_t nb = std::min(block, n - first), last = first + nb - 1, rest = n - last - 1, nb2 = std::min(block, rest);
+            // the second stream's update by panel p - 2 covers this panel's columns
+            if (lookahead && p >= 2) HIPCHK(hipStreamWaitEvent(s, updated[p & 1], 0));
+            HIPCHK(mfk::chol_step(N, s, a, n, first, (int)nb, (int)std::min(block, first), diag, st));
+            if (rest <= nb2) continue;
+            if (lookahead) {
+                HIPCHK(hipEventRecord(h->ev_panel, s));
+                HIPCHK(hipStreamWaitEvent(s1, h->ev_panel, 0));
+            }
+            // it skips its work only for failures in panels up to this one (a
+            // failure in a later panel comes after this update in MFLA's order)
+            const int64_t rest2 = rest - nb2;
+            const DV B21 = sub(a, last + 1 + nb2, first);
+            mfk::TileArgs u{};
+            u.mode = mfk::MODE_AB; u.net = mf::NET_STD; u.lower = 1; u.beta_zero = 0; u.tile = c.gemm_tile;
+            u.row_lo = 0; u.rows = rest2; u.n = rest2; u.K = nb; u.status_limit = last + 1;
+            HIPCHK(mfk::tile_launch_n(N, s1, u, B21, DV{B21.p, B21.cs, B21.rs, B21.ls}, sub(a, last + 1 + nb2, last + 1 + nb2), kMinusOne,
+                                      kOne, st));
+            if (lookahead) HIPCHK(hipEventRecord(updated[p & 1], s1));
+        }
+        HIPCHK(mfk::chol_diag_store(N, s, a, n, (int)block, diag, st));
+    } else
     for (int64_t first = 0; first < n; first += block) {
         const int64_t last = std::min(first + block, n) - 1, nb = last - first + 1;
         HIPCHK(mfk::chol_panel(N, s, a, first, last, st));

@@ -102,6 +102,164 @@ __global__ __launch_bounds__(256, 8) void k_chol_panel_lds(DV A, int64_t first, 
     }
 }
 
+// One step of the default factorization (panels of up to 16 columns): the
+// previous panel's update of this block column, the diagonal block and the
+// rows below it in one kernel. A panel's floor is its chain of 16 square
+// roots, divisions and products (x4: 6780 + 3560 + 916 cycles each, 75 us);
+// as three kernels (update, diagonal block, triangular solve) it took 13 +
+// 117 + 43 us and two more launches on that chain; one step takes 95-101 us.
+// x4 n = 256 / 1024 / 2048 / 4096: 2.91 / 12.3 / 27.2 / 104.5 ms -> 1.78 / 7.33 /
+// 20.6 / 101.8; x2 n = 1024 3.03 -> 2.04.
+//  * Every workgroup factors the diagonal block itself, in wave 0: element
+//    (r, c) keeps its running value in a lane (two slots a lane for columns 1
+//    to 5) and takes term k as soon as column k is final, with no barrier on
+//    the chain; the columns are published in LDS.
+//  * Waves 1-3 (a SIMD each, beside wave 0's) take 4 R rows each, a lane per
+//    (row, column): when column k is published the row's quotient by the
+//    pivot, then its term in the row's later columns: 4476 R cycles a column
+//    against wave 0's 11300, so the rows end one division after the block.
+// Per element the operations and their order are those of syrk! (alpha = -1,
+// beta = 1), the panel and trsm! (cholesky.jl:10-107). The diagonal block's
+// input is read by every workgroup, so its factor goes to `diag` and
+// chol_diag_store brings it home at the end; rows below hold their updated
+// values until the block has succeeded, as MFLA leaves them on failure.
+// A failure recorded by another workgroup of this step does not stop the
+// others (their rows' updates come before it in MFLA's order).
+constexpr int CS_B = 16, CS_FAIL = 1 << 20;
+
+template <int N, int R>
+__global__ __launch_bounds__(256) void k_chol_step(DV A, int64_t n, int64_t first, int nb, int np, double *diag, Status *st) {
+    __builtin_amdgcn_s_setprio(3);
+    const int64_t info = st->info;
+    if (info < 0 || (info > 0 && info <= first)) return;
+    constexpr int ROWS = 12 * R;
+    __shared__ __align__(16) double L[CS_B * CS_B * N];      // column-major: updated block, then its factor column by column
+    __shared__ __align__(16) double Pd[CS_B * CS_B * N];     // the previous panel, rows of the block: [k][row]
+    __shared__ __align__(16) double Pr[CS_B * ROWS * N];     // and this workgroup's rows
+    __shared__ __align__(16) double piv[N + 1];
+    __shared__ int cnt;                                      // columns published, or CS_FAIL
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    const int64_t r0 = first + nb + (int64_t)blockIdx.x * ROWS, pf = first - np;
+    // element idx of the columns c, c + 1, .. (len, len - 1, .. rows each)
+    auto packed = [](int idx, int c, int len, int &r, int &col) {
+        while (idx >= len) { idx -= len; ++c; --len; }
+        col = c;
+        r = c + idx;
+    };
+    for (int e = t; e < CS_B * np; e += 256) {
+        const int c = e % CS_B, k = e / CS_B;
+        if (c < nb) lds_put<N>(&Pd[e * N], ld<N>(A, first + c, pf + k));
+    }
+    for (int e = t; e < ROWS * np; e += 256) {
+        const int i = e % ROWS, k = e / ROWS;
+        if (r0 + i < n) lds_put<N>(&Pr[e * N], ld<N>(A, r0 + i, pf + k));
+    }
+    int dr = CS_B, dc = 0;
+    if (t < CS_B * (CS_B + 1) / 2) packed(t, 0, CS_B, dr, dc);
+    mf::V<N> d = dr < nb ? ld<N>(A, first + dr, first + dc) : mf::zero<N>();
+    // a row wave's elements: rows r0 + i0 + 4 q, column lc
+    const int lc = lane & 15, i0 = (wave - 1) * 4 * R + (lane >> 4);
+    mf::V<N> v[R];
+#pragma unroll
+    for (int q = 0; q < R; ++q) v[q] = wave > 0 && lc < nb && r0 + i0 + 4 * q < n ? ld<N>(A, r0 + i0 + 4 * q, first + lc) : mf::zero<N>();
+    if (t == 0) cnt = 0;
+    __syncthreads();
+    const mf::V<N> mone = mf::from<N>(-1.0), one = mf::from<N>(1.0);
+    auto updated = [&](const mf::V<N> &c, const double *row, int stride, int col) {
+        if (np == 0) return c;
+        mf::V<N> acc = mf::zero<N>();
+        for (int k = 0; k < np; ++k) acc = mf::mac(acc, lds_get<N>(row + k * stride * N), lds_get<N>(&Pd[(k * CS_B + col) * N]));
+        return mf::add(mf::mul(mone, acc), mf::mul(one, c));
+    };
+    if (dr < nb) lds_put<N>(&L[(dc * CS_B + dr) * N], updated(d, &Pd[dr * N], CS_B, dc));
+    __syncthreads();
+    if (wave == 0) {
+        // slot 0: columns 6..15 (55 elements) and the first 9 of columns
+        // 1..5, slot 1 the other 56 of those; column 0 has no terms
+        int er[3], ec[3];
+        mf::V<N> w[3];
+        if (lane < 55) packed(lane, 6, 10, er[0], ec[0]);
+        else packed(lane - 55, 1, 15, er[0], ec[0]);
+        er[1] = CS_B; ec[1] = -1;
+        if (lane < 56) packed(lane + 9, 1, 15, er[1], ec[1]);
+        er[2] = lane < CS_B ? lane : CS_B; ec[2] = lane < CS_B ? 0 : -1;
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+            if (er[q] >= nb) ec[q] = -1;
+            w[q] = ec[q] >= 0 ? lds_get<N>(&L[(ec[q] * CS_B + er[q]) * N]) : mf::zero<N>();
+        }
+        if (lane == 0) lds_put<N>(piv, w[2]);
+        for (int k = 0; k < nb; ++k) {
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+            const mf::V<N> dk = lds_get<N>(piv);
+            if (!mf::gt(dk, mf::zero<N>())) {
+                if (lane == 0) {
+                    __hip_atomic_store(&cnt, CS_FAIL, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
+                    if (blockIdx.x == 0) st->info = first + k + 1;
+                }
+                break;
+            }
+            const mf::V<N> p = mf::sqrt(dk);
+            const bool in0 = ec[0] == k, in1 = ec[1] == k, in2 = ec[2] == k;
+            const mf::V<N> x = in0 ? w[0] : (in1 ? w[1] : w[2]);
+            const int r = in0 ? er[0] : (in1 ? er[1] : er[2]);
+            mf::V<N> y = mf::div(x, p);
+            if (r == k) y = p;
+            if (in0 || in1 || in2) lds_put<N>(&L[(k * CS_B + r) * N], y);
+            if (lane == 0) __hip_atomic_store(&cnt, k + 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+            if (ec[0] > k) w[0] = mf::msub(w[0], lds_get<N>(&L[(k * CS_B + er[0]) * N]), lds_get<N>(&L[(k * CS_B + ec[0]) * N]));
+            if (k < 5 && ec[1] > k) w[1] = mf::msub(w[1], lds_get<N>(&L[(k * CS_B + er[1]) * N]), lds_get<N>(&L[(k * CS_B + ec[1]) * N]));
+            if (ec[0] == k + 1 && er[0] == k + 1) lds_put<N>(piv, w[0]);
+            if (ec[1] == k + 1 && er[1] == k + 1) lds_put<N>(piv, w[1]);
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+        if (blockIdx.x == 0) {
+            for (int e = lane; e < CS_B * CS_B; e += 64) {
+                const int r = e % CS_B, c = e / CS_B;
+                if (r >= c && r < nb) lds_put<N>(diag + (first * CS_B + e) * N, lds_get<N>(&L[e * N]));
+            }
+        }
+        return;
+    }
+#pragma unroll
+    for (int q = 0; q < R; ++q) {
+        const int i = i0 + 4 * q;
+        if (lc >= nb || r0 + i >= n) continue;
+        v[q] = updated(v[q], &Pr[i * N], ROWS, lc);
+        if (np > 0) stv<N>(A, r0 + i, first + lc, v[q]);
+    }
+    for (int k = 0; k < nb; ++k) {
+        int have;
+        while ((have = __hip_atomic_load(&cnt, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP)) <= k) __builtin_amdgcn_s_sleep(1);
+        if (have == CS_FAIL) return;
+        const mf::V<N> p = lds_get<N>(&L[(k * CS_B + k) * N]), a = lds_get<N>(&L[(k * CS_B + lc) * N]);
+#pragma unroll
+        for (int q = 0; q < R; ++q) {
+            mf::V<N> x;
+#pragma unroll
+            for (int l = 0; l < N; ++l) x.x[l] = __shfl(v[q].x[l], (lane & 48) + k, 64);
+            x = mf::div(x, p);
+            if (lc == k) v[q] = x;
+            else if (lc > k) v[q] = mf::msub(v[q], x, a);
+        }
+    }
+#pragma unroll
+    for (int q = 0; q < R; ++q)
+        if (lc < nb && r0 + i0 + 4 * q < n) stv<N>(A, r0 + i0 + 4 * q, first + lc, v[q]);
+}
+
+// The diagonal blocks' factors from k_chol_step's buffer: of every panel that
+// ran (those starting at or before a recorded failure).
+template <int N>
+__global__ void k_chol_diag_store(DV A, int64_t n, int block, const double *diag, const Status *st) {
+    const int64_t first = (int64_t)blockIdx.x * block, info = st->info;
+    if (info < 0 || (info > 0 && info <= first)) return;
+    const int r = threadIdx.x % CS_B, c = threadIdx.x / CS_B;
+    if (r < c || r >= block || first + r >= n) return;
+    stv<N>(A, first + r, first + c, lds_get<N>(diag + (first * CS_B + threadIdx.x) * N));
+}
+
 // Panels wider than 32 columns: the same computation from global memory.
 template <int N>
 __global__ __launch_bounds__(256) void k_chol_panel(DV A, int64_t first, int64_t last, Status *st) {
@@ -1363,6 +1521,44 @@ __global__ void k_fill_u8(uint8_t *p, int64_t n, uint8_t v) {
     }
 static inline unsigned nb(int64_t work, int b) { return (unsigned)cdiv(work > 0 ? work : 1, b); }
 template <int N> static S<N> mk(const double *v) { S<N> s; for (int l = 0; l < N; ++l) s.x[l] = v[l]; return s; }
+
+size_t chol_step_doubles(int N, int64_t n) { return (size_t)N * n * CS_B; }
+
+// Rows per wave: 4, or 8 from 3072 rows on (a workgroup per CU either way, so
+// that no two diagonal waves share a SIMD).
+hipError_t chol_step(int N, hipStream_t s, const DV &A, int64_t n, int64_t first, int nb, int np, double *diag, Status *st) {
+    if (nb < 1 || nb > CS_B || np < 0 || np > CS_B || first < np) return hipErrorInvalidValue;
+    const int64_t rest = n - first - nb;
+    const bool wide = rest > 12 * 256;
+    const int64_t groups = rest > 0 ? cdiv(rest, wide ? 24 : 12) : 1;
+    const dim3 grid((unsigned)groups);
+    auto launch = [&](auto ntag) {
+        constexpr int NN = decltype(ntag)::value;
+        if (wide) hipLaunchKernelGGL((k_chol_step<NN, 2>), grid, dim3(256), 0, s, A, n, first, nb, np, diag, st);
+        else hipLaunchKernelGGL((k_chol_step<NN, 1>), grid, dim3(256), 0, s, A, n, first, nb, np, diag, st);
+    };
+    switch (N) {
+        case 1: launch(std::integral_constant<int, 1>()); break;
+        case 2: launch(std::integral_constant<int, 2>()); break;
+        case 3: launch(std::integral_constant<int, 3>()); break;
+        case 4: launch(std::integral_constant<int, 4>()); break;
+        default: return hipErrorInvalidValue;
+    }
+    return hipGetLastError();
+}
+
+hipError_t chol_diag_store(int N, hipStream_t s, const DV &A, int64_t n, int block, const double *diag, const Status *st) {
+    if (block < 1 || block > CS_B) return hipErrorInvalidValue;
+    const dim3 grid((unsigned)cdiv(n, block));
+    switch (N) {
+        case 1: hipLaunchKernelGGL(k_chol_diag_store<1>, grid, dim3(256), 0, s, A, n, block, diag, st); break;
+        case 2: hipLaunchKernelGGL(k_chol_diag_store<2>, grid, dim3(256), 0, s, A, n, block, diag, st); break;
+        case 3: hipLaunchKernelGGL(k_chol_diag_store<3>, grid, dim3(256), 0, s, A, n, block, diag, st); break;
+        case 4: hipLaunchKernelGGL(k_chol_diag_store<4>, grid, dim3(256), 0, s, A, n, block, diag, st); break;
+        default: return hipErrorInvalidValue;
+    }
+    return hipGetLastError();
+}
 
 hipError_t chol_panel(int N, hipStream_t s, const DV &A, int64_t first, int64_t last, Status *st) {
     if (last - first + 1 <= 16) {

@@ -5,6 +5,13 @@
 namespace mfk {
 
 hipError_t chol_panel(int N, hipStream_t s, const DV &A, int64_t first, int64_t last, Status *st);
+// One step of a Cholesky factorization in panels of at most 16 columns: the
+// update of columns [first, first + nb) by the np columns before them, the
+// diagonal block (its factor to `diag`, chol_step_doubles(N, n) doubles) and
+// the rows below. chol_diag_store writes the diagonal blocks home at the end.
+size_t chol_step_doubles(int N, int64_t n);
+hipError_t chol_step(int N, hipStream_t s, const DV &A, int64_t n, int64_t first, int nb, int np, double *diag, Status *st);
+hipError_t chol_diag_store(int N, hipStream_t s, const DV &A, int64_t n, int block, const double *diag, const Status *st);
 // Pivot of column k over rows k..m-1; the row interchange is applied to the
 // panel columns [c0, c1) only (lu_laswp brings it to the other columns).
 hipError_t lu_pivot_swap(int N, hipStream_t s, const DV &A, int64_t k, int64_t m, int64_t c0, int64_t c1, int64_t *ipiv, Status *st);
