@@ -250,6 +250,18 @@ hipError_t ensure_side(mfla_handle h) {
 // panel_cus <= C keeps every bit inside its XCD's block. Fails (and the
 // caller runs without look-ahead) on a device without eight XCDs of at
 // least 16 CUs.
+// CUs the stream's kernels may run on (its mask; the device's where it has none)
+int64_t stream_cus(mfla_handle h, hipStream_t s) {
+    int cus = 0;
+    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, h->device) != hipSuccess) return 0;
+    uint32_t mask[32] = {};
+    const uint32_t words = (uint32_t)std::min(32, (cus + 31) / 32);
+    if (hipExtStreamGetCUMask(s, words, mask) != hipSuccess) { (void)hipGetLastError(); return cus; }
+    int64_t set = 0;
+    for (uint32_t w = 0; w < words; ++w) set += __builtin_popcount(mask[w]);
+    return set > 0 ? std::min<int64_t>(set, cus) : cus;
+}
+
 // CUs of ldlt! look-ahead's panel stream (four per XCD; the panels use at
 // most 32 workgroups there, and the first part of each update runs beside them)
 constexpr int kLdltPanelCUs = 32;
@@ -976,6 +988,10 @@ int mfla_getrf(mfla_handle h, int N, mfla_matrix A, int64_t *ipiv, double *origm
     if (int rc = original_maximum(h, N, A, 0, om)) return rc;
     const int64_t block = std::max<int64_t>(c.lu_block, 1);
     const DV a = dvn(A);
+    const int64_t panel_groups = 2 * stream_cus(h, s);   // lu_panel's workgroups, all resident at once
+    double *pbuf = (double *)grow_scratch(h, mfk::lu_panel_doubles() * sizeof(double));   // after original_maximum's use of it
+    if (!pbuf) return fail(MFLA_ERR_HIP, "scratch allocation failed");
+    HIPCHK(mfk::zero_fill(1, s, (int64_t)mfk::lu_panel_doubles(), 1, DV{pbuf, 1, 0, 0}));
     // Blocked right-looking LU (lu.jl:128-195). Row interchanges reach the
     // columns outside the current panel once the panel is done (lu_laswp),
     // before anything reads them. With look-ahead, the trsm!/gemm! update of
@@ -1006,9 +1022,13 @@ int mfla_getrf(mfla_handle h, int N, mfla_matrix A, int64_t *ipiv, double *origm
     };
     for (int64_t first = 0; first < kmax; first += block) {
         const int64_t last = std::min(first + block, kmax) - 1;
-        for (int64_t k = first; k <= last; ++k) {
-            HIPCHK(mfk::lu_pivot_swap(N, s, a, k, m, first, last + 1, ipiv, st));
-            HIPCHK(mfk::lu_scale_update(N, s, a, k, last, m, st));
+        if (block <= 16 && m - first <= mfk::lu_panel_max_rows() && mfk::lu_panel_workgroups(m - first) <= panel_groups) {
+            HIPCHK(mfk::lu_panel(N, s, a, first, (int)(last - first + 1), m, ipiv, pbuf, st));
+        } else {
+            for (int64_t k = first; k <= last; ++k) {
+                HIPCHK(mfk::lu_pivot_swap(N, s, a, k, m, first, last + 1, ipiv, st));
+                HIPCHK(mfk::lu_scale_update(N, s, a, k, last, m, st));
+            }
         }
         if (side_pending) {   // the previous trailing update owns the columns right of the next panel
             HIPCHK(hipStreamWaitEvent(s, h->ev_update, 0));
@@ -1038,6 +1058,7 @@ int mfla_getrf(mfla_handle h, int N, mfla_matrix A, int64_t *ipiv, double *origm
     }
     const int64_t r = read_info(h);
     if (r == INT64_MIN) return fail(MFLA_ERR_HIP, "status read failed");
+    if (r == -2) return fail(MFLA_ERR_HIP, "lu! panel: a workgroup waited for another past its bound");
     *info = r;
     for (int l = 0; l < N; ++l) origmax[l] = (r == -1) ? 0.0 : om[l];
     return MFLA_OK;
@@ -1373,6 +1394,7 @@ static int sytrf_run(mfla_handle h, int N, const mfla_matrix &A, const mfla_matr
     }
     const int64_t r = read_info(h);
     if (r == INT64_MIN) return fail(MFLA_ERR_HIP, "status read failed");
+    if (r == -2) return fail(MFLA_ERR_HIP, "lu! panel: a workgroup waited for another past its bound");
     *info = r;
     for (int l = 0; l < N; ++l) origmax[l] = (r == -1) ? 0.0 : om[l];
     return MFLA_OK;

@@ -467,6 +467,155 @@ __global__ __launch_bounds__(256, 8) void k_lu_scale_update(DV A, int64_t k, int
     if (j == 0) stv<N>(A, r, k, l);
 }
 
+// A whole panel of at most 16 columns in one kernel (lu.jl:34-82, 91-109) over
+// G workgroups, its elements in registers: a lane per (row, column), RPT rows
+// a thread, workgroup g's rows first + 16 (q G + g) + 0..15. Per column:
+//  * wave 0 takes the workgroup's first strict maximum and publishes it with
+//    that row's 16 values (workgroup 0, which owns the panel's first 16 rows,
+//    row k's values too), then reads every workgroup's, takes the same winner
+//    (largest value, then smallest row: any order gives it), fetches its row
+//    and forms the pivot's inverse;
+//  * all threads: rows k and p exchanged, l = a(r, k) inv, a(r, c) -= l u(c).
+// As two kernels per column (search and interchange, scaling and update) a
+// column took 9.4 us of kernels and 8 us between them; here 7.1 (x4 n = 512)
+// to 8.8 us (x3 n = 1999, beside the trailing update). x4 n = 256 / 1024 /
+// 2048 / 4096: 3.64 / 15.2 / 38.6 / 193.6 ms -> 2.61 / 11.5 / 34.8 / 188.3; x2 2.25
+// / 9.13 / 19.6 / 52.6 -> 1.56 / 7.08 / 16.0 / 46.4.
+//
+// The exchange goes through agent-scope atomics (written through, read past
+// the L2s), the data before the tag by a wait for the stores: a release or
+// acquire fence would write back and drop the L2 lines of the trailing update
+// beside it, every column. Tags hold the column's number + 1; the two buffers
+// alternate, and a workgroup writes one again only after every workgroup has
+// published the column in between, i.e. has read it. The G workgroups need
+// not start together, only to be resident together in the end (128 of the
+// chip's 256 CUs, whatever runs beside them ends by itself); a wait is bounded
+// all the same: past it st->info = kGridTimeout and the call fails.
+constexpr int LU_B = 16, LU_MAXG = 128, LU_SLOT = 72;   // slot: N limbs, row, (at 8) 16 N values
+constexpr int64_t kGridTimeout = -2;      // st->info after a bounded wait ended
+
+__device__ __forceinline__ void put_through(double *p, double x) {
+    __hip_atomic_store(reinterpret_cast<unsigned long long *>(p), __builtin_bit_cast(unsigned long long, x), __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ double get_through(const double *p) {
+    return __builtin_bit_cast(double, __hip_atomic_load(reinterpret_cast<const unsigned long long *>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+}
+
+template <int N, int RPT>
+__global__ __launch_bounds__(256, 4) void k_lu_panel(DV A, int64_t first, int nb, int64_t m, int64_t *ipiv, double *slots, double *krows,
+                                                     unsigned long long *tags, Status *st) {
+    __builtin_amdgcn_s_setprio(3);
+    if (st->info != 0) return;      // of an earlier kernel: none of this one is recorded before every workgroup has started
+    constexpr int LD = LU_B * N + 2;
+    __shared__ __align__(16) double R[LU_B * RPT * LD];     // the rows, as of this column
+    __shared__ __align__(16) double pr[LU_B * N], kr[LU_B * N], iv[N];
+    __shared__ int prow, bad;                               // pivot row - first; 1: zero pivot, 2: a wait ended
+    const int t = threadIdx.x, lane = t & 63, c = t & 15, ri = t >> 4, G = gridDim.x, g = blockIdx.x;
+    const int rows = (int)(m - first);
+    auto off = [&](int q) { return (q * G + g) * LU_B + ri; };   // row - first
+    mf::V<N> v[RPT];
+#pragma unroll
+    for (int q = 0; q < RPT; ++q) v[q] = off(q) < rows && c < nb ? ld<N>(A, first + off(q), first + c) : mf::zero<N>();
+    for (int k = 0; k < nb; ++k) {
+        const int64_t col = first + k;
+#pragma unroll
+        for (int q = 0; q < RPT; ++q) lds_put<N>(&R[(q * LU_B + ri) * LD + c * N], v[q]);
+        __syncthreads();
+        if (t < 64) {
+            mf::V<N> best = mf::zero<N>();
+            best.x[0] = -1.0;                               // below every |a|; a NaN never replaces it
+            int bi = INT32_MAX;
+            if (lane < LU_B * RPT) {
+                const int r = ((lane / LU_B) * G + g) * LU_B + lane % LU_B;
+                if (r >= k && r < rows) {
+                    mf::V<N> x = mf::vabs(lds_get<N>(&R[lane * LD + k * N]));
+                    // MFLA's scan keeps a NaN in row k: nothing compares above it
+                    if (r == k && __builtin_isnan(x.x[0])) { _Pragma("unroll") for (int l = 0; l < N; ++l) x.x[l] = __builtin_inf(); }
+                    if (mf::gt(x, best)) { best = x; bi = r; }
+                }
+            }
+            lp_wave_argmax<N>(best, bi);
+            double *slot = slots + ((k & 1) * LU_MAXG + g) * LU_SLOT, *krow = krows + (k & 1) * LU_SLOT;
+            if (bi != INT32_MAX) {
+                const int i = (bi / (LU_B * G)) * LU_B + bi % LU_B;
+                if (lane < LU_B * N) put_through(slot + 8 + lane, R[i * LD + lane]);
+            }
+            if (g == 0 && lane < LU_B * N) put_through(krow + lane, R[k * LD + lane]);
+#pragma unroll
+            for (int l = 0; l < N; ++l)
+                if (lane == l) put_through(slot + l, best.x[l]);
+            if (lane == N) put_through(slot + N, (double)bi);
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            if (lane == 0) __hip_atomic_store(tags + g, (unsigned long long)(col + 1), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            bool all = false;
+            for (unsigned spins = 0; spins < (1u << 22); ++spins) {
+                bool here = true;
+                for (int j = lane; j < G; j += 64)
+                    here = here && __hip_atomic_load(tags + j, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= (unsigned long long)(col + 1);
+                if (__builtin_amdgcn_ballot_w64(!here) == 0) { all = true; break; }
+                __builtin_amdgcn_s_sleep(1);
+            }
+            asm volatile("" ::: "memory");
+            best = mf::zero<N>();
+            best.x[0] = -1.0;
+            bi = INT32_MAX;
+            const double *other = slots + (k & 1) * LU_MAXG * LU_SLOT;
+            for (int j = lane; j < G; j += 64) {
+                mf::V<N> x;
+#pragma unroll
+                for (int l = 0; l < N; ++l) x.x[l] = get_through(other + j * LU_SLOT + l);
+                const int xi = (int)get_through(other + j * LU_SLOT + N);
+                if (xi != INT32_MAX && (mf::gt(x, best) || (mf::eq(x, best) && xi < bi))) { best = x; bi = xi; }
+            }
+            lp_wave_argmax<N>(best, bi);
+            const double *from = other + ((bi / LU_B) % G) * LU_SLOT + 8;
+            if (bi == INT32_MAX) { bi = k; from = krow; }   // nothing compared: row k stays
+            if (lane < LU_B * N) {
+                pr[lane] = get_through(from + lane);
+                kr[lane] = get_through(krow + lane);
+            }
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+            const mf::V<N> piv = lds_get<N>(&pr[k * N]);
+            const bool zero = mf::is_zero(piv);
+            const mf::V<N> inv = mf::inv(piv);
+            if (lane == 0) {
+                lds_put<N>(iv, inv);
+                prow = bi;
+                bad = !all ? 2 : (zero ? 1 : 0);
+                if (g == 0 && all) ipiv[col] = first + bi + 1;
+                if (!all) st->info = kGridTimeout;
+                else if (g == 0 && zero) st->info = col + 1;
+            }
+        }
+        __syncthreads();
+        const int p = prow, stop = bad;
+        if (stop == 2) return;
+        const mf::V<N> u = lds_get<N>(&pr[c * N]), inv = lds_get<N>(iv);
+#pragma unroll
+        for (int q = 0; q < RPT; ++q) {
+            const int r = off(q);
+            if (r == p) v[q] = lds_get<N>(&kr[c * N]);
+            if (r == k) v[q] = u;
+        }
+        if (stop) break;
+#pragma unroll
+        for (int q = 0; q < RPT; ++q) {
+            const int r = off(q);
+            mf::V<N> x;
+#pragma unroll
+            for (int l = 0; l < N; ++l) x.x[l] = __shfl(v[q].x[l], (lane & 48) + k, 64);
+            if (r <= k || r >= rows) continue;
+            const mf::V<N> lk = mf::mul(x, inv);
+            if (c == k) v[q] = lk;
+            else if (c > k) v[q] = mf::msub(v[q], lk, u);
+        }
+    }
+#pragma unroll
+    for (int q = 0; q < RPT; ++q)
+        if (off(q) < rows && c < nb) stv<N>(A, first + off(q), first + c, v[q]);
+}
+
 // Sequential row interchanges on right-hand sides (solve.jl:85-113).
 template <int N>
 __global__ void k_apply_ipiv(DV B, int64_t count, int64_t nrhs, const int64_t *ipiv) {
@@ -897,7 +1046,6 @@ __global__ __launch_bounds__(512) void k_ldlt_panel(DV A, int64_t n, int64_t pfi
 constexpr int GP_T = 192;                 // row threads per workgroup
 constexpr int GP_THREADS = GP_T + 64;     // and the helper wave (one wave per SIMD)
 constexpr int GP_MAXG = 64;               // workgroups per launch (co-resident)
-constexpr int64_t kGridTimeout = -2;      // st->info after a barrier timed out
 
 __host__ __device__ constexpr size_t ldlt_grid_partials(int N) { return (size_t)GP_MAXG * (2 * (N + 1) + N + 1); }
 
@@ -1567,6 +1715,41 @@ hipError_t chol_panel(int N, hipStream_t s, const DV &A, int64_t first, int64_t 
         MF_DISPATCH(N, hipLaunchKernelGGL((k_chol_panel_lds<NN, CHOL_LDS>), dim3(1), dim3(256), 0, s, A, first, last, st));
     } else {
         MF_DISPATCH(N, hipLaunchKernelGGL(k_chol_panel<NN>, dim3(1), dim3(256), 0, s, A, first, last, st));
+    }
+    return hipGetLastError();
+}
+
+size_t lu_panel_doubles() { return (size_t)(2 * LU_MAXG + 2) * LU_SLOT + LU_MAXG; }
+
+int64_t lu_panel_max_rows() { return (int64_t)LU_MAXG * LU_B * 4; }
+
+// Workgroups of 16 rows up to 128 of them, then two or four rows a thread
+// (`buf`'s tags are zero before a factorization's first panel).
+static int lu_rows_per_thread(int64_t rows) {
+    const int64_t blocks = cdiv(rows, LU_B);
+    return blocks <= LU_MAXG ? 1 : (blocks <= 2 * LU_MAXG ? 2 : 4);
+}
+int64_t lu_panel_workgroups(int64_t rows) { return cdiv(cdiv(rows, LU_B), lu_rows_per_thread(rows)); }
+
+hipError_t lu_panel(int N, hipStream_t s, const DV &A, int64_t first, int nb, int64_t m, int64_t *ipiv, double *buf, Status *st) {
+    const int64_t rows = m - first;
+    if (nb < 1 || nb > LU_B || rows < nb || rows > lu_panel_max_rows()) return hipErrorInvalidValue;
+    const int rpt = lu_rows_per_thread(rows);
+    const dim3 grid((unsigned)lu_panel_workgroups(rows));
+    double *krows = buf + (size_t)2 * LU_MAXG * LU_SLOT;
+    unsigned long long *tags = reinterpret_cast<unsigned long long *>(krows + 2 * LU_SLOT);
+    auto launch = [&](auto ntag) {
+        constexpr int NN = decltype(ntag)::value;
+        if (rpt == 1) hipLaunchKernelGGL((k_lu_panel<NN, 1>), grid, dim3(256), 0, s, A, first, nb, m, ipiv, buf, krows, tags, st);
+        else if (rpt == 2) hipLaunchKernelGGL((k_lu_panel<NN, 2>), grid, dim3(256), 0, s, A, first, nb, m, ipiv, buf, krows, tags, st);
+        else hipLaunchKernelGGL((k_lu_panel<NN, 4>), grid, dim3(256), 0, s, A, first, nb, m, ipiv, buf, krows, tags, st);
+    };
+    switch (N) {
+        case 1: launch(std::integral_constant<int, 1>()); break;
+        case 2: launch(std::integral_constant<int, 2>()); break;
+        case 3: launch(std::integral_constant<int, 3>()); break;
+        case 4: launch(std::integral_constant<int, 4>()); break;
+        default: return hipErrorInvalidValue;
     }
     return hipGetLastError();
 }

@@ -12,6 +12,13 @@ hipError_t chol_panel(int N, hipStream_t s, const DV &A, int64_t first, int64_t 
 size_t chol_step_doubles(int N, int64_t n);
 hipError_t chol_step(int N, hipStream_t s, const DV &A, int64_t n, int64_t first, int nb, int np, double *diag, Status *st);
 hipError_t chol_diag_store(int N, hipStream_t s, const DV &A, int64_t n, int block, const double *diag, const Status *st);
+// A panel of nb <= 16 columns with its pivots (ipiv) and, within the panel,
+// its interchanges, for at most lu_panel_max_rows() rows first..m-1; buf:
+// lu_panel_doubles() doubles, zero before a factorization's first panel.
+size_t lu_panel_doubles();
+int64_t lu_panel_max_rows();
+int64_t lu_panel_workgroups(int64_t rows);   // they wait for each other: all have to be resident
+hipError_t lu_panel(int N, hipStream_t s, const DV &A, int64_t first, int nb, int64_t m, int64_t *ipiv, double *buf, Status *st);
 // Pivot of column k over rows k..m-1; the row interchange is applied to the
 // panel columns [c0, c1) only (lu_laswp brings it to the other columns).
 hipError_t lu_pivot_swap(int N, hipStream_t s, const DV &A, int64_t k, int64_t m, int64_t c0, int64_t c1, int64_t *ipiv, Status *st);
