@@ -30,57 +30,7 @@
 namespace mfk {
 
 constexpr int TB = 64;   // diagonal block rows (threads in x)
-constexpr int TC = 4;    // right-hand sides per workgroup (threads in y)
 
-template <int N, bool FWD>
-__global__ __launch_bounds__(TB *TC) void k_trsm_diag(int64_t p0, int nbk, int64_t nrhs, DV X, DV CA, DV D, int unit,
-                                                      int swap, const Status *st, int64_t lim) {
-    if (st && st->info != 0 && (lim == 0 || st->info < 0 || st->info <= lim)) return;
-    __shared__ double xs[TC * N];
-    const int tx = threadIdx.x, ty = threadIdx.y;
-    const int64_t c = (int64_t)blockIdx.x * TC + ty;
-    const bool valid = (tx < nbk) && (c < nrhs);
-    const int64_t p = p0 + tx;
-    mf::V<N> v = valid ? ld<N>(X, p, c) : mf::zero<N>();
-    for (int s0 = 0; s0 < nbk; ++s0) {
-        const int s = FWD ? s0 : nbk - 1 - s0;
-        const int64_t q = p0 + s;
-        if (tx == s && valid) {
-            if (!unit) v = mf::div(v, ld<N>(D, q, q));
-            stv<N>(X, q, c, v);
-#pragma unroll
-            for (int l = 0; l < N; ++l) xs[ty * N + l] = v.x[l];
-        }
-        __syncthreads();
-        if (valid && (FWD ? tx > s : tx < s)) {
-            mf::V<N> xq;
-#pragma unroll
-            for (int l = 0; l < N; ++l) xq.x[l] = xs[ty * N + l];
-            v = swap ? mf::msub(v, xq, ld<N>(CA, p, q)) : mf::msub(v, ld<N>(CA, p, q), xq);
-        }
-        __syncthreads();
-    }
-}
-
-// The same diagonal-block solve without barriers: a group of G lanes holds
-// one right-hand side (lane p_local = unknown p0 + p_local). At step s the
-// owner lane's running value is final; the group reads it by shuffle and
-// every lane of the group forms the same quotient x_s (so no lane waits for
-// another), then the later unknowns subtract their term. Per element the
-// operations and their order are those of k_trsm_diag.
-//
-// With look-ahead these solves run beside the side stream's tile updates:
-// held to 64 VGPRs (8 waves per SIMD; 80 for four limbs, whose previous-block
-// terms would spill otherwise) they fit next to the update's waves, and their
-// raised wave priority lets the SIMD issue them first.
-//
-// The serial chain waits on no global load: the block's diagonal is staged
-// in LDS once (all groups of the workgroup share the block), and each step's
-// coefficient CA(p, q) is loaded before the step's division -- one step
-// ahead for up to three limbs; at the top of the step for four, where a
-// second coefficient in registers would spill under the 64-VGPR bound. The
-// loads use a row index clamped into the block (lanes that do not use the
-// value read an in-bounds entry they ignore).
 // Start mark for the side stream: *start_sig = start_value from thread 0 of
 // every workgroup (the same value; any one suffices). A kernel starts only
 // after the kernel before it on its stream has ended and released its
@@ -102,24 +52,22 @@ __device__ __forceinline__ double group_bcast(double x, int grp, int s) {
     }
 }
 
-//
-// With K > 0 the kernel first subtracts the K terms of the block solved just
-// before (unknowns q0 .. q0 + K - 1, ascending q: the order and operations of
-// the MODE_SUB tile update it replaces), so that update is not a kernel of
-// its own on the serial chain of blocks.
-//
-// With far_flag the kernel first waits (bounded) for *far_flag >= far_wait:
-// the side stream's update that last reaches this block's rows was enqueued
-// before this kernel and waits only for kernels before it, so the wait ends;
-// past the bound the block's values are written as NaN and *err = 1.
+// Blocks of up to 32 unknowns without look-ahead (the panels' solves): a group
+// of G lanes holds one right-hand side (lane p_local = unknown p0 + p_local).
+// At step s the owner lane's running value is final; the group reads it by
+// shuffle and every lane of the group forms the same quotient x_s (so no lane
+// waits for another), then the later unknowns subtract their term (MFLA's
+// order and operations). Held to 64 VGPRs (80 for four limbs) with raised wave
+// priority: the panels' solves run beside a trailing update. The block's
+// diagonal is staged in LDS once; each step's coefficient is loaded before the
+// step's division, one step ahead for up to three limbs. The loads use a row
+// index clamped into the block (lanes that do not use the value read an
+// in-bounds entry they ignore).
 template <int N, bool FWD, int G>
 __global__ __launch_bounds__(256, N == 4 ? 5 : 8) void k_trsm_diag_wave(int64_t p0, int nbk, int64_t nrhs, DV X, DV CA, DV D, int unit, int swap,
-                                                           const Status *st, int64_t lim, int64_t q0, int K, const unsigned *far_flag,
-                                                           unsigned far_wait, unsigned *err, unsigned *start_sig, unsigned start_value) {
+                                                                       const Status *st, int64_t lim) {
     __builtin_amdgcn_s_setprio(3);
-    mark_start(start_sig, start_value);
     if (st && st->info != 0 && (lim == 0 || st->info < 0 || st->info <= lim)) return;
-    const bool ok = far_flag == nullptr || wait_flag(far_flag, far_wait);
     __shared__ double dg[G * N];
     constexpr int RPW = 64 / G;
     const int lane = threadIdx.x & 63, grp = lane / G, pl = lane % G;
@@ -130,25 +78,6 @@ __global__ __launch_bounds__(256, N == 4 ? 5 : 8) void k_trsm_diag_wave(int64_t 
     if (!unit && (int)threadIdx.x < nbk) lds_put<N>(&dg[threadIdx.x * N], ld<N>(D, p0 + threadIdx.x, p0 + threadIdx.x));
     constexpr bool kAhead = N <= 3;
     mf::V<N> v = valid ? ld<N>(X, p, c) : mf::zero<N>();
-    if (!ok) {
-#pragma unroll
-        for (int l = 0; l < N; ++l) v.x[l] = __builtin_nan("");
-        if (threadIdx.x == 0) __hip_atomic_store(err, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-    if (K > 0) {
-        // terms of the previous block (every lane computes; invalid lanes'
-        // values are never stored), the next term's operands loaded ahead
-        const int64_t cc = c < nrhs ? c : nrhs - 1;
-        mf::V<N> an2 = ld<N>(CA, pc, q0), xn2 = ld<N>(X, q0, cc);
-        for (int k = 0; k < K; ++k) {
-            const mf::V<N> a = an2, xq = xn2;
-            if (k + 1 < K) {
-                an2 = ld<N>(CA, pc, q0 + k + 1);
-                xn2 = ld<N>(X, q0 + k + 1, cc);
-            }
-            v = swap ? mf::msub(v, xq, a) : mf::msub(v, a, xq);
-        }
-    }
     mf::V<N> an = kAhead ? ld<N>(CA, pc, p0 + (FWD ? 0 : nbk - 1)) : mf::zero<N>();
     __syncthreads();
     for (int s0 = 0; s0 < nbk; ++s0) {
@@ -173,6 +102,110 @@ __global__ __launch_bounds__(256, N == 4 ? 5 : 8) void k_trsm_diag_wave(int64_t 
                 v = swap ? mf::msub(v, xq, a) : mf::msub(v, a, xq);
             }
         }
+    }
+}
+
+// A diagonal block of up to 64 unknowns, a wave per right-hand side (lane =
+// unknown, the operations and order of k_trsm_diag_wave) and the coefficients
+// through LDS: the workgroup's four waves share them, CH columns at a time,
+// the next CH loading into registers meanwhile. A step is one division and one
+// product (x2 0.3 us, x4 1.9), and a coefficient loaded one step ahead by each
+// wave made it wait for memory instead (a 4096-unknown solve, x2 256 right-hand sides
+// 4.41 -> 3.81 ms, x2 64 backward 3.75 -> 3.14, x4 64 backward 12.4 -> 11.9, x4
+// 64 forward 11.8 -> 10.9 with the faster division, x3 and x4 256 unchanged).
+//
+// With K > 0 the kernel first subtracts the K <= 64 terms of the block solved
+// just before (unknowns q0 .. q0 + K - 1, ascending q: the order and operations
+// of the MODE_SUB tile update it replaces), so that update is not a kernel of
+// its own on the serial chain of blocks; their coefficients are the first K
+// columns of the same stream.
+//
+// With far_flag the kernel first waits (bounded) for *far_flag >= far_wait:
+// the side stream's update that last reaches this block's rows was enqueued
+// before this kernel and waits only for kernels before it, so the wait ends;
+// past the bound the block's values are written as NaN and *err = 1.
+template <int N, bool FWD>
+__global__ __launch_bounds__(256, N == 4 ? 4 : 6) void k_trsm_diag_lds(int64_t p0, int nbk, int64_t nrhs, DV X, DV CA, DV D, int unit, int swap,
+                                                                      const Status *st, int64_t lim, int64_t q0, int K, const unsigned *far_flag,
+                                                                      unsigned far_wait, unsigned *err, unsigned *start_sig, unsigned start_value) {
+    __builtin_amdgcn_s_setprio(3);
+    mark_start(start_sig, start_value);
+    if (st && st->info != 0 && (lim == 0 || st->info < 0 || st->info <= lim)) return;
+    constexpr int CH = N <= 2 ? 16 : 8, E = TB * CH / 256, LD = TB * N + 2;   // padded: column-wise writes spread over the banks
+    __shared__ double cf[2][CH * LD];          // [column][limb][row]
+    __shared__ __align__(16) double dg[TB * N];
+    __shared__ __align__(16) double xs[4 * TB * N];
+    const int t = threadIdx.x, lane = t & 63, w = t >> 6, T = K + nbk;
+    const int64_t c = (int64_t)blockIdx.x * 4 + w, cc = c < nrhs ? c : nrhs - 1, p = p0 + lane;
+    const bool valid = lane < nbk && c < nrhs;
+    const bool colfast = CA.cs == 1 && CA.rs != 1;
+    auto place = [&](int q, int &row, int &col) {
+        const int e = t + 256 * q;
+        if (colfast) { col = e % CH; row = e / CH; } else { row = e % TB; col = e / TB; }
+    };
+    mf::V<N> pre[E];
+    auto fetch = [&](int j0) {                 // columns j0 .. j0 + CH - 1 of the stream, rows and columns clamped into it
+#pragma unroll
+        for (int q = 0; q < E; ++q) {
+            int row, col;
+            place(q, row, col);
+            const int j = j0 + col < T ? j0 + col : T - 1, r = row < nbk ? row : nbk - 1;
+            pre[q] = ld<N>(CA, p0 + r, j < K ? q0 + j : p0 + (FWD ? j - K : nbk - 1 - (j - K)));
+        }
+    };
+    auto stage = [&](double *to) {
+#pragma unroll
+        for (int q = 0; q < E; ++q) {
+            int row, col;
+            place(q, row, col);
+#pragma unroll
+            for (int l = 0; l < N; ++l) to[col * LD + l * TB + row] = pre[q].x[l];
+        }
+    };
+    fetch(0);
+    if (!unit && t < nbk) lds_put<N>(&dg[t * N], ld<N>(D, p0 + t, p0 + t));
+    if (lane < K) lds_put<N>(&xs[(w * TB + lane) * N], ld<N>(X, q0 + lane, cc));
+    const bool ok = far_flag == nullptr || wait_flag(far_flag, far_wait);
+    mf::V<N> v = valid ? ld<N>(X, p, c) : mf::zero<N>();
+    if (!ok) {
+#pragma unroll
+        for (int l = 0; l < N; ++l) v.x[l] = __builtin_nan("");
+        if (t == 0) __hip_atomic_store(err, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    stage(cf[0]);
+    if (CH < T) fetch(CH);
+    __syncthreads();
+    for (int j0 = 0, b = 0; j0 < T; j0 += CH, b ^= 1) {
+        const int m = T - j0 < CH ? T - j0 : CH;
+        for (int i = 0; i < m; ++i) {
+            const int j = j0 + i;
+            mf::V<N> a;
+#pragma unroll
+            for (int l = 0; l < N; ++l) a.x[l] = cf[b][i * LD + l * TB + lane];
+            if (j < K) {
+                const mf::V<N> xq = lds_get<N>(&xs[(w * TB + j) * N]);
+                v = swap ? mf::msub(v, xq, a) : mf::msub(v, a, xq);
+                continue;
+            }
+            const int s = FWD ? j - K : nbk - 1 - (j - K);
+            mf::V<N> xq;
+#pragma unroll
+            for (int l = 0; l < N; ++l) xq.x[l] = group_bcast<64>(v.x[l], 0, s);
+            if (!unit) xq = mf::div(xq, lds_get<N>(&dg[s * N]));
+            if (valid) {
+                if (lane == s) {
+                    v = xq;
+                    stv<N>(X, p, c, xq);
+                } else if (FWD ? lane > s : lane < s) {
+                    v = swap ? mf::msub(v, xq, a) : mf::msub(v, a, xq);
+                }
+            }
+        }
+        if (j0 + CH < T) {
+            stage(cf[b ^ 1]);
+            if (j0 + 2 * CH < T) fetch(j0 + 2 * CH);
+        }
+        __syncthreads();
     }
 }
 
@@ -389,26 +422,26 @@ template <int N>
 static hipError_t diag(hipStream_t s, bool fwd, int64_t p0, int nbk, int64_t nrhs, const DV &X, const DV &CA, const DV &D, int unit,
                        int swap, const Status *st, int64_t lim, int64_t q0 = 0, int K = 0, const unsigned *far_flag = nullptr,
                        unsigned far_wait = 0, unsigned *err = nullptr, unsigned *start_sig = nullptr, unsigned start_value = 0) {
+    if (nbk < 1 || nbk > TB || K < 0 || K > TB) return hipErrorInvalidValue;
+    if (nbk > 32 || K > 0 || far_flag || start_sig) {
+        const dim3 grid((unsigned)cdiv(nrhs, 4));
+        if (fwd)
+            hipLaunchKernelGGL((k_trsm_diag_lds<N, true>), grid, dim3(256), 0, s, p0, nbk, nrhs, X, CA, D, unit, swap, st, lim, q0, K, far_flag,
+                               far_wait, err, start_sig, start_value);
+        else
+            hipLaunchKernelGGL((k_trsm_diag_lds<N, false>), grid, dim3(256), 0, s, p0, nbk, nrhs, X, CA, D, unit, swap, st, lim, q0, K, far_flag,
+                               far_wait, err, start_sig, start_value);
+        return hipGetLastError();
+    }
     // one group of G lanes per right-hand side, 4 waves per workgroup
     auto launch = [&](auto gtag) {
         constexpr int G = decltype(gtag)::value;
         const dim3 grid((unsigned)cdiv(cdiv(nrhs, 64 / G), 4)), block(256);
-        if (fwd)
-            hipLaunchKernelGGL((k_trsm_diag_wave<N, true, G>), grid, block, 0, s, p0, nbk, nrhs, X, CA, D, unit, swap, st, lim, q0, K, far_flag,
-                               far_wait, err, start_sig, start_value);
-        else
-            hipLaunchKernelGGL((k_trsm_diag_wave<N, false, G>), grid, block, 0, s, p0, nbk, nrhs, X, CA, D, unit, swap, st, lim, q0, K, far_flag,
-                               far_wait, err, start_sig, start_value);
+        if (fwd) hipLaunchKernelGGL((k_trsm_diag_wave<N, true, G>), grid, block, 0, s, p0, nbk, nrhs, X, CA, D, unit, swap, st, lim);
+        else hipLaunchKernelGGL((k_trsm_diag_wave<N, false, G>), grid, block, 0, s, p0, nbk, nrhs, X, CA, D, unit, swap, st, lim);
     };
-    if ((far_flag || start_sig) && nbk > TB) return hipErrorInvalidValue;
     if (nbk <= 16) launch(std::integral_constant<int, 16>());
-    else if (nbk <= 32) launch(std::integral_constant<int, 32>());
-    else if (nbk <= TB) launch(std::integral_constant<int, 64>());
-    else {
-        dim3 grid((unsigned)cdiv(nrhs, TC)), block(TB, TC);
-        if (fwd) hipLaunchKernelGGL((k_trsm_diag<N, true>), grid, block, 0, s, p0, nbk, nrhs, X, CA, D, unit, swap, st, lim);
-        else hipLaunchKernelGGL((k_trsm_diag<N, false>), grid, block, 0, s, p0, nbk, nrhs, X, CA, D, unit, swap, st, lim);
-    }
+    else launch(std::integral_constant<int, 32>());
     return hipGetLastError();
 }
 
