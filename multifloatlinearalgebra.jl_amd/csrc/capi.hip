@@ -348,7 +348,7 @@ constexpr int64_t kTrsmWaitMaxRhs = 256;
 
 // trsm! core (trsm.jl:247-301) after argument checks; alpha scaling included.
 hipError_t trsm_core(mfla_handle h, int N, int side, int uplo, int trans, int diag, const mfla_matrix &B, const mfla_matrix &A,
-                     const double *alpha, const mfla_config &c, const Status *st) {
+                     const double *alpha, const mfla_config &c, const Status *st, bool lower_rhs = false) {   // lower_rhs: B lower triangular, a forward solve
     const int64_t n = A.rows;
     if (alpha && !scalar_is_one(alpha, N)) {
         hipError_t e = mfk::scale(N, h->stream, B.rows, B.cols, dvn(B), alpha, st);
@@ -360,6 +360,7 @@ hipError_t trsm_core(mfla_handle h, int N, int side, int uplo, int trans, int di
     a.n = n;
     a.unit = diag == MFLA_UNIT;
     a.exact_order = trsm_exact(c, n) ? 1 : 0;
+    a.lower_rhs = lower_rhs;
     a.swap_product = side == MFLA_RIGHT ? 1 : 0;   // B[i,k]*coeff(k,j) (trsm.jl:136-172)
     DV X, CA;
     if (side == MFLA_LEFT) {
@@ -388,7 +389,7 @@ hipError_t trsm_core(mfla_handle h, int N, int side, int uplo, int trans, int di
         // 12.6 ms, x2 4.3 -> 3.7 ms), a loss where the updates are (256
         // right-hand sides and more; x3, whose updates cost more beside its
         // chain: 7.5 -> 7.8 ms).
-        a.stream_next = a.forward && a.nrhs <= kTrsmStreamMaxRhs && N != 3;
+        a.stream_next = a.forward && a.nrhs <= kTrsmStreamMaxRhs && N != 3 && !a.lower_rhs;
         // Up to 256 right-hand sides each diagonal kernel waits for the side
         // stream's updates on the same device words instead of the stream
         // waiting on events (4096 x 256: x4 forward 19.9 -> 19.6 ms, backward
@@ -2237,8 +2238,15 @@ int check_adjoint_factor(int N, const mfla_matrix &F, int64_t info) {
 }
 
 // S^{-1} B in place from the Cholesky factor (the potrs path)
-hipError_t potrs_core(mfla_handle h, int N, const mfla_matrix &F, const mfla_matrix &B, const mfla_config &c) {
-    hipError_t e = trsm_core(h, N, MFLA_LEFT, MFLA_LOWER, MFLA_NOTRANS, MFLA_NONUNIT, B, F, kOne, c, nullptr);
+// B = S^{-1} B with S = L L'. The adjoints have no order of MFLA's to keep, so
+// where the caller leaves the order open their solves take the blocked one at
+// every size (the exact one, the default up to n = 256, is a chain of n^2/2
+// terms). lower: B is lower triangular, so the forward solve's rows end at
+// their block's last column (n^3/6 products for n^3/2; the same bits).
+hipError_t potrs_core(mfla_handle h, int N, const mfla_matrix &F, const mfla_matrix &B, const mfla_config &config, bool lower = false) {
+    mfla_config c = config;
+    if (c.trsm_order == MFLA_TRSM_ORDER_AUTO) c.trsm_order = MFLA_TRSM_ORDER_BLOCKED;
+    hipError_t e = trsm_core(h, N, MFLA_LEFT, MFLA_LOWER, MFLA_NOTRANS, MFLA_NONUNIT, B, F, kOne, c, nullptr, lower);
     if (e != hipSuccess) return e;
     return trsm_core(h, N, MFLA_LEFT, MFLA_LOWER, MFLA_TRANS, MFLA_NONUNIT, B, F, kOne, c, nullptr);
 }
@@ -2307,7 +2315,7 @@ int mfla_logdet_adjoint(mfla_handle h, int N, mfla_matrix F, int64_t info, const
     std::lock_guard<std::mutex> g(h->lock);
     hipStream_t s = h->stream;
     HIPCHK(mfk::identity(N, s, n, dvn(Sbar)));
-    HIPCHK(potrs_core(h, N, F, Sbar, c));                                    // S^{-1}
+    HIPCHK(potrs_core(h, N, F, Sbar, c, true));                              // S^{-1}
     double half_ybar[4] = {0.0, 0.0, 0.0, 0.0};
     for (int l = 0; l < N; ++l) half_ybar[l] = 0.5 * ybar[l];
     HIPCHK(mfk::symmetrize(N, s, n, dvn(Sbar), dvn(Sbar), half_ybar));     // ybar * sym(S^{-1})

@@ -465,8 +465,12 @@ static hipError_t solve_t(hipStream_t s, const TrsmArgs &a, const DV &X, const D
         if (rows <= 0) return hipSuccess;
         TileArgs u = t;
         u.rows = rows; u.K = K;
+        if (a.lower_rhs && q0 + K < nrhs) u.n = q0 + K;   // the block's rows are zero beyond
         return tile_launch_n(N, ss, u, sub(CA, r0, q0), sub(X, q0, 0), sub(X, r0, 0), nullptr, nullptr, st);
     };
+    if (a.lower_rhs && !a.forward) return hipErrorInvalidValue;
+    // right-hand sides of the block of rows ending before p1
+    auto upto = [&](int64_t p1) { return a.lower_rhs && p1 < nrhs ? p1 : nrhs; };
     // Look-ahead (blocked orders, n > 3 blocks, a side stream): the terms of
     // block b reach the rows of block b + 1 in the next block's diagonal
     // kernel (its prologue), and the rows beyond on the side stream while
@@ -550,7 +554,7 @@ static hipError_t solve_t(hipStream_t s, const TrsmArgs &a, const DV &X, const D
             auto block_step = [&](int64_t p0, int nbk, int64_t far0, int64_t nfar) -> hipError_t {
                 hipError_t q;
                 const unsigned wait = (b >= 2 && had_far[b & 1]) ? b - 1 : 0;
-                if ((q = diag<N>(s, a.forward != 0, p0, nbk, nrhs, X, CA, D, a.unit, a.swap_product, st, a.status_limit, prev0, prevK,
+                if ((q = diag<N>(s, a.forward != 0, p0, nbk, upto(p0 + nbk), X, CA, D, a.unit, a.swap_product, st, a.status_limit, prev0, prevK,
                                  wait ? a.far_flag : nullptr, wait, a.far_flag + 1, a.start_sig, b)) != hipSuccess)
                     return q;
                 if (pend.rows > 0) {
@@ -604,7 +608,7 @@ static hipError_t solve_t(hipStream_t s, const TrsmArgs &a, const DV &X, const D
                 if ((r = hipStreamWaitEvent(s, far_ev[slot], 0)) != hipSuccess) return r;
                 far_pending[slot] = false;
             }
-            if ((r = diag<N>(s, a.forward != 0, p0, nbk, nrhs, X, CA, D, a.unit, a.swap_product, st, a.status_limit, prev0, prevK)) !=
+            if ((r = diag<N>(s, a.forward != 0, p0, nbk, upto(p0 + nbk), X, CA, D, a.unit, a.swap_product, st, a.status_limit, prev0, prevK)) !=
                 hipSuccess)
                 return r;
             if (nfar > 0) {
@@ -641,7 +645,7 @@ static hipError_t solve_t(hipStream_t s, const TrsmArgs &a, const DV &X, const D
     if (a.forward) {
         for (int64_t p0 = 0; p0 < n; p0 += TB) {
             const int nbk = (int)((n - p0) < TB ? (n - p0) : TB);
-            if ((e = diag<N>(s, true, p0, nbk, nrhs, X, CA, D, a.unit, a.swap_product, st, a.status_limit)) != hipSuccess) return e;
+            if ((e = diag<N>(s, true, p0, nbk, upto(p0 + nbk), X, CA, D, a.unit, a.swap_product, st, a.status_limit)) != hipSuccess) return e;
             const int64_t p1 = p0 + nbk;
             if (p1 < n && (e = update(s, p1, n - p1, p0, nbk)) != hipSuccess) return e;
         }
@@ -651,7 +655,7 @@ static hipError_t solve_t(hipStream_t s, const TrsmArgs &a, const DV &X, const D
     for (int64_t p1 = n; p1 > 0; p1 -= TB) {
         const int64_t p0 = p1 > TB ? p1 - TB : 0;
         const int nbk = (int)(p1 - p0);
-        if ((e = diag<N>(s, false, p0, nbk, nrhs, X, CA, D, a.unit, a.swap_product, st, a.status_limit)) != hipSuccess) return e;
+        if ((e = diag<N>(s, false, p0, nbk, upto(p0 + nbk), X, CA, D, a.unit, a.swap_product, st, a.status_limit)) != hipSuccess) return e;
         if (p0 > 0 && (e = update(s, 0, p0, p0, nbk)) != hipSuccess) return e;
     }
     return hipSuccess;

@@ -31,6 +31,9 @@ struct TrsmArgs {
     // With far_flag: a device word each diagonal kernel marks at its start
     // (block b's far update waits for block b + 1's mark on the side stream).
     unsigned *start_sig;
+    // Forward: the right-hand sides are a lower triangular matrix, so each
+    // block of rows takes the columns up to its last row (the rest are zero).
+    int lower_rhs;
     // The caller's stream and `side` have hardware queues of their own (so
     // a kernel on one may wait for work enqueued after it on the other).
     int dedicated;
