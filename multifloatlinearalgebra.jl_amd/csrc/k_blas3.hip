@@ -197,8 +197,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 8))) voi
             }
         }
         const int kend = (K - k0) < BK ? (int)(K - k0) : BK;
-        for (int kk = 0; kk < kend; ++kk) {
-            mf::V<N> av[TM], bv[TN];
+        auto read = [&](int kk, mf::V<N> (&av)[TM], mf::V<N> (&bv)[TN]) {
 #pragma unroll
             for (int a = 0; a < TM; ++a)
 #pragma unroll
@@ -207,6 +206,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 8))) voi
             for (int b = 0; b < TN; ++b)
 #pragma unroll
                 for (int l = 0; l < N; ++l) bv[b].x[l] = Bs[b_slot(kk, ty * TN + b) + l];
+        };
+        auto step = [&](const mf::V<N> (&av)[TM], const mf::V<N> (&bv)[TN]) {
 #pragma unroll
             for (int a = 0; a < TM; ++a)
 #pragma unroll
@@ -214,6 +215,29 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 8))) voi
                     if (MODE == MODE_SUB) acc[a][b] = swap ? mf::msub(acc[a][b], bv[b], av[a]) : mf::msub(acc[a][b], av[a], bv[b]);
                     else acc[a][b] = mf::Mac<N, NET>::apply(acc[a][b], av[a], bv[b]);
                 }
+        };
+        if constexpr (TM * TN == 1 && MODE == MODE_AB && !LOWER) {
+            // one element a thread: the next k's operands are read while this
+            // one's product is summed, two k a turn (a wave alone on its SIMD
+            // otherwise waits for LDS at every k: x4 256^3 148 -> 142 us, 100 x
+            // 300 x 100 174 -> 160; the triangular solves' updates, four waves on
+            // a SIMD, lose by the registers: x4 4096 x 256 18.9 -> 20.0 ms)
+            mf::V<N> a0[TM], b0[TN], a1[TM], b1[TN];
+            read(0, a0, b0);
+            int kk = 0;
+            for (; kk + 1 < kend; kk += 2) {
+                read(kk + 1, a1, b1);
+                step(a0, b0);
+                read(kk + 2 < BK ? kk + 2 : BK - 1, a0, b0);
+                step(a1, b1);
+            }
+            if (kk < kend) step(a0, b0);
+        } else {
+            for (int kk = 0; kk < kend; ++kk) {
+                mf::V<N> av[TM], bv[TN];
+                read(kk, av, bv);
+                step(av, bv);
+            }
         }
         __syncthreads();
     }
