@@ -1035,19 +1035,22 @@ int mfla_getrf(mfla_handle h, int N, mfla_matrix A, int64_t *ipiv, double *origm
             HIPCHK(hipStreamWaitEvent(s, h->ev_update, 0));
             side_pending = false;
         }
-        HIPCHK(mfk::lu_laswp(N, s, a, first, last - first + 1, ipiv, 0, first, last + 1, n - last - 1));
-        if (last + 1 >= n) continue;
-        const int64_t rest = n - last - 1, nxt = std::min(block, rest);
+        const int64_t nb = last - first + 1, rest = n - last - 1, nxt = std::min(block, std::max<int64_t>(rest, 0));
         if (!lookahead || rest <= nxt || last + 1 >= kmax) {
-            HIPCHK(update(s, first, last, last + 1, rest, 0));
+            HIPCHK(mfk::lu_laswp(N, s, a, first, nb, ipiv, 0, first, last + 1, rest));
+            if (rest > 0) HIPCHK(update(s, first, last, last + 1, rest, 0));
             continue;
         }
-        HIPCHK(hipEventRecord(h->ev_panel, s));
-        HIPCHK(update(s, first, last, last + 1, nxt, 0));
-        // the rest on the side stream; it skips its work only for failures in
+        // On the chain only the next panel's columns: their interchanges and
+        // their update. The other columns' interchanges and the rest of the
+        // update on the side stream; it skips its work only for failures in
         // panels up to this one (a later failure comes after this update in
         // MFLA's order)
+        HIPCHK(hipEventRecord(h->ev_panel, s));
+        HIPCHK(mfk::lu_laswp(N, s, a, first, nb, ipiv, 0, 0, last + 1, nxt));
+        HIPCHK(update(s, first, last, last + 1, nxt, 0));
         HIPCHK(hipStreamWaitEvent(s1, h->ev_panel, 0));
+        HIPCHK(mfk::lu_laswp(N, s1, a, first, nb, ipiv, 0, first, last + 1 + nxt, rest - nxt));
         HIPCHK(update(s1, first, last, last + 1 + nxt, rest - nxt, last + 1));
         HIPCHK(hipEventRecord(h->ev_update, s1));
         side_pending = true;
