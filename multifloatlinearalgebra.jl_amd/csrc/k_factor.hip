@@ -516,8 +516,8 @@ __global__ __launch_bounds__(256, 8) void k_lu_scale_update(DV A, int64_t k, int
 // beside it, every column. Tags hold the column's number + 1; the two buffers
 // alternate, and a workgroup writes one again only after every workgroup has
 // published the column in between, i.e. has read it. The G workgroups need
-// not start together, only to be resident together in the end (128 of the
-// chip's 256 CUs, whatever runs beside them ends by itself); a wait is bounded
+// not start together, only to be resident together in the end (at most 128 on
+// the chip's 256 CUs, whatever runs beside them ends by itself); a wait is bounded
 // all the same: past it st->info = kGridTimeout and the call fails.
 constexpr int LU_B = 16, LU_MAXG = 128, LU_SLOT = 72;   // slot: N limbs, row, (at 8) 16 N values
 constexpr int64_t kGridTimeout = -2;      // st->info after a bounded wait ended
@@ -1751,11 +1751,13 @@ size_t lu_panel_doubles() { return (size_t)(2 * LU_MAXG + 2) * LU_SLOT + LU_MAXG
 
 int64_t lu_panel_max_rows() { return (int64_t)LU_MAXG * LU_B * 4; }
 
-// Workgroups of 16 rows up to 128 of them, then two or four rows a thread
-// (`buf`'s tags are zero before a factorization's first panel).
+// Workgroups of 16 rows up to 64 of them, then two or four rows a thread (128
+// of one row each are slower to exchange than two rows a thread to compute:
+// x2 n = 2048 14.9 -> 13.8 ms). `buf`'s tags are zero before a factorization's
+// first panel.
 static int lu_rows_per_thread(int64_t rows) {
     const int64_t blocks = cdiv(rows, LU_B);
-    return blocks <= LU_MAXG ? 1 : (blocks <= 2 * LU_MAXG ? 2 : 4);
+    return blocks <= LU_MAXG / 2 ? 1 : (blocks <= LU_MAXG ? 2 : 4);
 }
 int64_t lu_panel_workgroups(int64_t rows) { return cdiv(cdiv(rows, LU_B), lu_rows_per_thread(rows)); }
 

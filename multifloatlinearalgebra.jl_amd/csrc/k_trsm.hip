@@ -59,37 +59,37 @@ __device__ __forceinline__ double group_bcast(double x, int grp, int s) {
 // waits for another), then the later unknowns subtract their term (MFLA's
 // order and operations). Held to 64 VGPRs (80 for four limbs) with raised wave
 // priority: the panels' solves run beside a trailing update. The block's
-// diagonal is staged in LDS once; each step's coefficient is loaded before the
-// step's division, one step ahead for up to three limbs. The loads use a row
-// index clamped into the block (lanes that do not use the value read an
-// in-bounds entry they ignore).
+// coefficients are staged in LDS once, as no step is long enough to hide a
+// load from memory behind it (lu!'s 16-unknown solves took 11.6 us with three
+// limbs and 19.6 with four; with half the panel's workgroups, lu! x3 n = 1999
+// 22.6 -> 21.9 ms, x2 n = 4096 44.0 -> 41.7).
 template <int N, bool FWD, int G>
 __global__ __launch_bounds__(256, N == 4 ? 5 : 8) void k_trsm_diag_wave(int64_t p0, int nbk, int64_t nrhs, DV X, DV CA, DV D, int unit, int swap,
                                                                        const Status *st, int64_t lim) {
     __builtin_amdgcn_s_setprio(3);
     if (st && st->info != 0 && (lim == 0 || st->info < 0 || st->info <= lim)) return;
-    __shared__ double dg[G * N];
+    __shared__ __align__(16) double dg[G * N];
+    __shared__ double cf[G * G * N];                     // [column][limb][row]
     constexpr int RPW = 64 / G;
-    const int lane = threadIdx.x & 63, grp = lane / G, pl = lane % G;
-    const int64_t c = ((int64_t)blockIdx.x * 4 + (threadIdx.x >> 6)) * RPW + grp;
+    const int t = threadIdx.x, lane = t & 63, grp = lane / G, pl = lane % G;
+    const int64_t c = ((int64_t)blockIdx.x * 4 + (t >> 6)) * RPW + grp;
     const bool valid = pl < nbk && c < nrhs;
-    const int64_t p = p0 + pl;
-    const int64_t pc = p0 + (pl < nbk ? pl : nbk - 1);   // in-bounds row for the unconditional loads
-    if (!unit && (int)threadIdx.x < nbk) lds_put<N>(&dg[threadIdx.x * N], ld<N>(D, p0 + threadIdx.x, p0 + threadIdx.x));
-    constexpr bool kAhead = N <= 3;
-    mf::V<N> v = valid ? ld<N>(X, p, c) : mf::zero<N>();
-    mf::V<N> an = kAhead ? ld<N>(CA, pc, p0 + (FWD ? 0 : nbk - 1)) : mf::zero<N>();
+    const bool colfast = CA.cs == 1 && CA.rs != 1;
+    for (int e = t; e < G * G; e += 256) {
+        const int row = colfast ? e / G : e % G, col = colfast ? e % G : e / G;
+        if (row >= nbk || col >= nbk) continue;
+        const mf::V<N> a = ld<N>(CA, p0 + row, p0 + col);
+#pragma unroll
+        for (int l = 0; l < N; ++l) cf[(col * N + l) * G + row] = a.x[l];
+    }
+    if (!unit && t < nbk) lds_put<N>(&dg[t * N], ld<N>(D, p0 + t, p0 + t));
+    mf::V<N> v = valid ? ld<N>(X, p0 + pl, c) : mf::zero<N>();
     __syncthreads();
     for (int s0 = 0; s0 < nbk; ++s0) {
         const int s = FWD ? s0 : nbk - 1 - s0;
-        const int64_t q = p0 + s;
         mf::V<N> a;
-        if constexpr (kAhead) {
-            a = an;
-            if (s0 + 1 < nbk) an = ld<N>(CA, pc, FWD ? q + 1 : q - 1);
-        } else {
-            a = ld<N>(CA, pc, q);
-        }
+#pragma unroll
+        for (int l = 0; l < N; ++l) a.x[l] = cf[(s * N + l) * G + pl];
         mf::V<N> xq;
 #pragma unroll
         for (int l = 0; l < N; ++l) xq.x[l] = group_bcast<G>(v.x[l], grp, s);
@@ -97,7 +97,7 @@ __global__ __launch_bounds__(256, N == 4 ? 5 : 8) void k_trsm_diag_wave(int64_t 
         if (valid) {
             if (pl == s) {
                 v = xq;
-                stv<N>(X, q, c, xq);
+                stv<N>(X, p0 + s, c, xq);
             } else if (FWD ? pl > s : pl < s) {
                 v = swap ? mf::msub(v, xq, a) : mf::msub(v, a, xq);
             }
