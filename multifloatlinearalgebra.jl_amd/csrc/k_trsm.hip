@@ -52,6 +52,34 @@ __device__ __forceinline__ double group_bcast(double x, int grp, int s) {
     }
 }
 
+// One step for one unknown's running value v: the quotient (stored to X(p, c))
+// if it is this unknown's, less the term if it comes later. Up to three limbs
+// by selects, every lane computing and storing its value once, at the end of
+// the block (solve_end): a branch costs a wave ~100 cycles (x2 1024 x 16 0.79
+// -> 0.68 ms, x3 1.65 -> 1.58). With four limbs the selects cost more (2.96 ->
+// 3.03 ms).
+template <int N>
+__device__ __forceinline__ void solve_step(mf::V<N> &v, const mf::V<N> &xq, const mf::V<N> &a, int swap, bool valid, bool own, bool later,
+                                           const DV &X, int64_t p, int64_t c) {
+    if constexpr (N == 4) {
+        if (valid) {
+            if (own) {
+                v = xq;
+                stv<N>(X, p, c, xq);
+            } else if (later) {
+                v = swap ? mf::msub(v, xq, a) : mf::msub(v, a, xq);
+            }
+        }
+    } else {
+        const mf::V<N> x = swap ? xq : a, y = swap ? a : xq, next = mf::msub(v, x, y);
+#pragma unroll
+        for (int l = 0; l < N; ++l) v.x[l] = own ? xq.x[l] : (later ? next.x[l] : v.x[l]);
+    }
+}
+template <int N> __device__ __forceinline__ void solve_end(const mf::V<N> &v, bool valid, const DV &X, int64_t p, int64_t c) {
+    if (N < 4 && valid) stv<N>(X, p, c, v);
+}
+
 // Blocks of up to 32 unknowns without look-ahead (the panels' solves): a group
 // of G lanes holds one right-hand side (lane p_local = unknown p0 + p_local).
 // At step s the owner lane's running value is final; the group reads it by
@@ -94,15 +122,9 @@ __global__ __launch_bounds__(256, N == 4 ? 5 : 8) void k_trsm_diag_wave(int64_t 
 #pragma unroll
         for (int l = 0; l < N; ++l) xq.x[l] = group_bcast<G>(v.x[l], grp, s);
         if (!unit) xq = mf::div(xq, lds_get<N>(&dg[s * N]));
-        if (valid) {
-            if (pl == s) {
-                v = xq;
-                stv<N>(X, p0 + s, c, xq);
-            } else if (FWD ? pl > s : pl < s) {
-                v = swap ? mf::msub(v, xq, a) : mf::msub(v, a, xq);
-            }
-        }
+        solve_step<N>(v, xq, a, swap, valid, pl == s, FWD ? pl > s : pl < s, X, p0 + s, c);
     }
+    solve_end<N>(v, valid, X, p0 + pl, c);
 }
 
 // A diagonal block of up to 64 unknowns, a wave per right-hand side (lane =
@@ -192,14 +214,7 @@ __global__ __launch_bounds__(256, N == 4 ? 4 : 6) void k_trsm_diag_lds(int64_t p
 #pragma unroll
             for (int l = 0; l < N; ++l) xq.x[l] = group_bcast<64>(v.x[l], 0, s);
             if (!unit) xq = mf::div(xq, lds_get<N>(&dg[s * N]));
-            if (valid) {
-                if (lane == s) {
-                    v = xq;
-                    stv<N>(X, p, c, xq);
-                } else if (FWD ? lane > s : lane < s) {
-                    v = swap ? mf::msub(v, xq, a) : mf::msub(v, a, xq);
-                }
-            }
+            solve_step<N>(v, xq, a, swap, valid, lane == s, FWD ? lane > s : lane < s, X, p, c);
         }
         if (j0 + CH < T) {
             stage(cf[b ^ 1]);
@@ -207,6 +222,7 @@ __global__ __launch_bounds__(256, N == 4 ? 4 : 6) void k_trsm_diag_lds(int64_t p
         }
         __syncthreads();
     }
+    solve_end<N>(v, valid, X, p, c);
 }
 
 // Forward look-ahead with the next block's rows streamed. A workgroup of 8
@@ -265,15 +281,9 @@ __global__ __launch_bounds__(512, N == 4 ? 3 : 4) void k_trsm_diag_stream(int64_
                 lds_put<N>(&xs[(r * 64 + s) * N], xq);
                 __hip_atomic_store(&cnt[r], s + 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
             }
-            if (valid) {
-                if (lane == s) {
-                    v = xq;
-                    stv<N>(X, q, c, xq);
-                } else if (lane > s) {
-                    v = swap ? mf::msub(v, xq, a) : mf::msub(v, a, xq);
-                }
-            }
+            solve_step<N>(v, xq, a, swap, valid, lane == s, lane > s, X, q, c);
         }
+        solve_end<N>(v, valid, X, p, c);
     } else {
         const bool valid = lane < nn && c < nrhs;
         const int64_t p = p1 + lane, pc = p1 + (lane < nn ? lane : nn - 1);
