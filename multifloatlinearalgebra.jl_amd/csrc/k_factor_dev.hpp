@@ -293,8 +293,13 @@ __device__ BKChoice wg_select_bk(int64_t n, int64_t k, const mf::V<N> &alpha, E 
     }
     const mf::V<N> rowmax = wg_max<N>(rm, sv_buf);
     if (mf::ge(absakk, mf::mul(mf::mul(alpha, colmax), mf::div(colmax, rowmax)))) return BKChoice{1, k};
-    if (mf::ge(mf::vabs(e.entry(imax, imax)), mf::mul(alpha, rowmax))) return BKChoice{1, imax};
-    return BKChoice{2, imax};
+    const bool one = mf::ge(mf::vabs(e.entry(imax, imax)), mf::mul(alpha, rowmax));
+    // The interchange that follows writes A(imax, imax): no wave may start it
+    // before every wave has read that element, or the waves' choices differ
+    // and their barriers no longer pair (an index then comes from another
+    // reduction's buffer).
+    __syncthreads();
+    return BKChoice{one ? 1 : 2, imax};
 }
 
 // Entries of the right-looking factorization: the trailing block is updated
