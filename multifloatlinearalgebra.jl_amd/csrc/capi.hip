@@ -37,6 +37,11 @@ struct mfla_handle_s {
     int *flags = nullptr;       // small device flag array
     void *scratch = nullptr;    // grows on demand (non-hot paths only)
     size_t scratch_bytes = 0;
+    // panel exchange of potrf / getrf, whose calls end with a status read: a
+    // buffer of its own, since an asynchronous call on another stream of the
+    // handle may still be reading scratch
+    void *panels = nullptr;
+    size_t panels_bytes = 0;
     std::mutex lock;            // calls on one handle are serialised
     hipStream_t side = nullptr; // second stream of the look-ahead factorization
     hipEvent_t ev_join = nullptr, ev_panel = nullptr, ev_update = nullptr, ev_update2 = nullptr;
@@ -148,16 +153,19 @@ const mfla_config &cfg_or_default(const mfla_config *c, mfla_config &tmp) {
     return tmp;
 }
 
-void *grow_scratch(mfla_handle h, size_t bytes) {
-    if (h->scratch_bytes < bytes) {
-        if (h->scratch) { (void)hipStreamSynchronize(h->stream); (void)hipFree(h->scratch); }
-        h->scratch = nullptr;
-        h->scratch_bytes = 0;
-        if (hipMalloc(&h->scratch, bytes) != hipSuccess) return nullptr;
-        h->scratch_bytes = bytes;
+void *grow(mfla_handle h, void *&buf, size_t &held, size_t bytes) {
+    if (held < bytes) {
+        if (buf) { (void)hipStreamSynchronize(h->stream); (void)hipFree(buf); }
+        buf = nullptr;
+        held = 0;
+        if (hipMalloc(&buf, bytes) != hipSuccess) return nullptr;
+        held = bytes;
     }
-    return h->scratch;
+    return buf;
 }
+
+void *grow_scratch(mfla_handle h, size_t bytes) { return grow(h, h->scratch, h->scratch_bytes, bytes); }
+void *grow_panels(mfla_handle h, size_t bytes) { return grow(h, h->panels, h->panels_bytes, bytes); }
 
 int64_t read_info(mfla_handle h, int64_t *aux = nullptr, hipStream_t on = nullptr) {
     Status local{};
@@ -532,6 +540,7 @@ int mfla_handle_destroy(mfla_handle h) {
     (void)hipFree(h->flags);
     if (h->pinned) (void)hipHostFree(h->pinned);
     if (h->scratch) (void)hipFree(h->scratch);
+    if (h->panels) (void)hipFree(h->panels);
     if (h->side) {
         (void)hipStreamSynchronize(h->side);
         (void)hipStreamDestroy(h->side);
@@ -894,7 +903,7 @@ int mfla_potrf(mfla_handle h, int N, mfla_matrix A, int64_t *info, const mfla_co
     // of its columns by the panel before, the panel, the rows below), the
     // update of the columns beyond the next panel on the second stream.
     if (block <= 16 && n > 0) {
-        double *diag = (double *)grow_scratch(h, mfk::chol_step_doubles(N, n) * sizeof(double));
+        double *diag = (double *)grow_panels(h, mfk::chol_step_doubles(N, n) * sizeof(double));
         if (!diag) return fail(MFLA_ERR_HIP, "scratch allocation failed");
         const hipEvent_t updated[2] = {h->ev_update, h->ev_update2};   // by the panel's parity
         int64_t p = 0;
@@ -990,7 +999,7 @@ int mfla_getrf(mfla_handle h, int N, mfla_matrix A, int64_t *ipiv, double *origm
     const int64_t block = std::max<int64_t>(c.lu_block, 1);
     const DV a = dvn(A);
     const int64_t panel_groups = 2 * stream_cus(h, s);   // lu_panel's workgroups, all resident at once
-    double *pbuf = (double *)grow_scratch(h, mfk::lu_panel_doubles() * sizeof(double));   // after original_maximum's use of it
+    double *pbuf = (double *)grow_panels(h, mfk::lu_panel_doubles() * sizeof(double));
     if (!pbuf) return fail(MFLA_ERR_HIP, "scratch allocation failed");
     HIPCHK(mfk::zero_fill(1, s, (int64_t)mfk::lu_panel_doubles(), 1, DV{pbuf, 1, 0, 0}));
     // Blocked right-looking LU (lu.jl:128-195). Row interchanges reach the
