@@ -248,16 +248,6 @@ hipError_t ensure_side(mfla_handle h) {
     return hipEventCreateWithFlags(&h->ev_update, hipEventDisableTiming);
 }
 
-// The CU-partitioned streams of ldlt!'s look-ahead (default priority):
-// panel_cus CUs for the panels, the device's other CUs for the trailing
-// updates, so a panel's latency-bound waves never share a SIMD with the
-// update's. Mask bit C x + 8 y + x (XCD x < 8, y < panel_cus / 8, C = CUs /
-// 8) gives each of the eight XCDs panel_cus / 8 of them whether the driver
-// maps mask bits to XCDs in blocks of C or in turn, so every XCD runs work
-// of both streams (a kernel's workgroups are dealt to the XCDs in turn);
-// panel_cus <= C keeps every bit inside its XCD's block. Fails (and the
-// caller runs without look-ahead) on a device without eight XCDs of at
-// least 16 CUs.
 // CUs the stream's kernels may run on (its mask; the device's where it has none)
 int64_t stream_cus(mfla_handle h, hipStream_t s) {
     int cus = 0;
@@ -270,6 +260,17 @@ int64_t stream_cus(mfla_handle h, hipStream_t s) {
     return set > 0 ? std::min<int64_t>(set, cus) : cus;
 }
 
+// The CU-partitioned streams of ldlt!'s look-ahead (default priority):
+// panel_cus CUs for the panels, the device's other CUs for the trailing
+// updates, so a panel's latency-bound waves never share a SIMD with the
+// update's. Mask bit C x + 8 y + x (XCD x < 8, y < panel_cus / 8, C = CUs /
+// 8) gives each of the eight XCDs panel_cus / 8 of them whether the driver
+// maps mask bits to XCDs in blocks of C or in turn, so every XCD runs work
+// of both streams (a kernel's workgroups are dealt to the XCDs in turn);
+// panel_cus <= C keeps every bit inside its XCD's block. Fails (and the
+// caller runs without look-ahead) on a device without eight XCDs of at
+// least 16 CUs.
+//
 // CUs of ldlt! look-ahead's panel stream (four per XCD; the panels use at
 // most 32 workgroups there, and the first part of each update runs beside them)
 constexpr int kLdltPanelCUs = 32;
@@ -346,6 +347,9 @@ bool trsm_exact(const mfla_config &c, int64_t n) {
         hipError_t e_ = (expr);             \
         if (e_ != hipSuccess) return e_;    \
     } while (0)
+
+// Status of a panel kernel whose bounded wait for another workgroup ended.
+constexpr int64_t kGridTimeoutInfo = -2;
 
 // Right-hand sides up to which a Float64x4 trsm_core look-ahead runs on the
 // CU-partitioned streams, up to which a forward one streams the next block's
@@ -1071,7 +1075,7 @@ int mfla_getrf(mfla_handle h, int N, mfla_matrix A, int64_t *ipiv, double *origm
     }
     const int64_t r = read_info(h);
     if (r == INT64_MIN) return fail(MFLA_ERR_HIP, "status read failed");
-    if (r == -2) return fail(MFLA_ERR_HIP, "lu! panel: a workgroup waited for another past its bound");
+    if (r == kGridTimeoutInfo) return fail(MFLA_ERR_HIP, "lu! panel: a workgroup waited for another past its bound");
     *info = r;
     for (int l = 0; l < N; ++l) origmax[l] = (r == -1) ? 0.0 : om[l];
     return MFLA_OK;
@@ -1120,7 +1124,6 @@ static size_t noalloc_layout(int N, int64_t n, const mfla_ldlt_plan_t &plan, siz
 // workgroups (0: the 512-thread single-workgroup kernel); every choice gives
 // the same bits.
 constexpr int64_t kLdltPanelRows = 192;
-constexpr int64_t kGridTimeoutInfo = -2;
 constexpr int64_t kLdltSpecMaxDepth = 32;
 static int64_t ldlt_panel_workgroup_cap() {
     const char *v = std::getenv("MFLA_LDLT_PANEL_WORKGROUPS");
@@ -1407,7 +1410,6 @@ static int sytrf_run(mfla_handle h, int N, const mfla_matrix &A, const mfla_matr
     }
     const int64_t r = read_info(h);
     if (r == INT64_MIN) return fail(MFLA_ERR_HIP, "status read failed");
-    if (r == -2) return fail(MFLA_ERR_HIP, "lu! panel: a workgroup waited for another past its bound");
     *info = r;
     for (int l = 0; l < N; ++l) origmax[l] = (r == -1) ? 0.0 : om[l];
     return MFLA_OK;
@@ -2249,12 +2251,12 @@ int check_adjoint_factor(int N, const mfla_matrix &F, int64_t info) {
     return MFLA_OK;
 }
 
-// S^{-1} B in place from the Cholesky factor (the potrs path)
-// B = S^{-1} B with S = L L'. The adjoints have no order of MFLA's to keep, so
-// where the caller leaves the order open their solves take the blocked one at
-// every size (the exact one, the default up to n = 256, is a chain of n^2/2
-// terms). lower: B is lower triangular, so the forward solve's rows end at
-// their block's last column (n^3/6 products for n^3/2; the same bits).
+// B = S^{-1} B with S = L L' (the potrs path). The adjoints have no order of
+// MFLA's to keep, so where the caller leaves the order open their solves take
+// the blocked one at every size (the exact one, the default up to n = 256, is
+// a chain of n^2/2 terms). lower: B is lower triangular, so the forward
+// solve's rows end at their block's last column (n^3/6 products for n^3/2; the
+// same bits).
 hipError_t potrs_core(mfla_handle h, int N, const mfla_matrix &F, const mfla_matrix &B, const mfla_config &config, bool lower = false) {
     mfla_config c = config;
     if (c.trsm_order == MFLA_TRSM_ORDER_AUTO) c.trsm_order = MFLA_TRSM_ORDER_BLOCKED;

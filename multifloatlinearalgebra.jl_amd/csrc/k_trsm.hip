@@ -233,7 +233,7 @@ __global__ __launch_bounds__(256, N == 4 ? 4 : 6) void k_trsm_diag_lds(int64_t p
 // far_wait, written after that update), subtract this block's terms in
 // ascending q as the solver waves publish them in LDS -- the operands,
 // operations and order of the next kernel's previous-block terms
-// (k_trsm_diag_wave with K > 0), which then has none. That update was
+// (k_trsm_diag_lds with K > 0), which then has none. That update was
 // enqueued before this kernel and waits only for the kernel before it, so
 // the wait ends; it is bounded all the same, and past the bound the rows
 // are written as NaN (and *err = 1) instead of values without the update.
@@ -665,7 +665,7 @@ static hipError_t solve_t(hipStream_t s, const TrsmArgs &a, const DV &X, const D
     for (int64_t p1 = n; p1 > 0; p1 -= TB) {
         const int64_t p0 = p1 > TB ? p1 - TB : 0;
         const int nbk = (int)(p1 - p0);
-        if ((e = diag<N>(s, false, p0, nbk, upto(p0 + nbk), X, CA, D, a.unit, a.swap_product, st, a.status_limit)) != hipSuccess) return e;
+        if ((e = diag<N>(s, false, p0, nbk, nrhs, X, CA, D, a.unit, a.swap_product, st, a.status_limit)) != hipSuccess) return e;
         if (p0 > 0 && (e = update(s, 0, p0, p0, nbk)) != hipSuccess) return e;
     }
     return hipSuccess;
