@@ -246,7 +246,13 @@ int mfla_symv(mfla_handle h, int limbs, int uplo, mfla_matrix y, mfla_matrix A, 
 /* ---------------------------------------------------- factorizations */
 /* cholesky! (src/factorizations/cholesky.jl:68-107): lower, in place */
 int mfla_potrf(mfla_handle h, int limbs, mfla_matrix A, int64_t *info, const mfla_config *config);
-/* lu! (src/factorizations/lu.jl:128-195): ipiv_dev has min(m, n) int64 */
+/* lu! (src/factorizations/lu.jl:128-195): ipiv_dev has min(m, n) int64.
+ * lu!'s and ldlt!'s panels wait across workgroups, so of the calls that run at
+ * once on a device (handles, threads) only as many as their streams' CUs hold
+ * take them; the others run slower panels with the same bits. Calls of another
+ * process on the same CUs are not seen: should they keep a panel's workgroups
+ * out past its bounded wait, the call returns MFLA_ERR_HIP with A partly
+ * factored. */
 int mfla_getrf(mfla_handle h, int limbs, mfla_matrix A, int64_t *ipiv_dev, double *original_maximum, int64_t *info,
                const mfla_config *config, mfla_workspace ws);
 /* ldlt! (src/factorizations/ldlt.jl:654-717): dsub is an n x 1 device matrix;

@@ -26,6 +26,7 @@
 #include "k_refine.hpp"
 #include "k_trsm.hpp"
 #include "mf_arith.hpp"
+#include "residency.hpp"
 
 using mfk::DV;
 using mfk::Status;
@@ -1002,7 +1003,16 @@ int mfla_getrf(mfla_handle h, int N, mfla_matrix A, int64_t *ipiv, double *origm
     if (int rc = original_maximum(h, N, A, 0, om)) return rc;
     const int64_t block = std::max<int64_t>(c.lu_block, 1);
     const DV a = dvn(A);
-    const int64_t panel_groups = 2 * stream_cus(h, s);   // lu_panel's workgroups, all resident at once
+    // lu_panel's workgroups wait for each other: at most two a CU (which holds
+    // four), and places for the largest panel or the column kernels instead
+    const int64_t cus = stream_cus(h, s);
+    int64_t panel_groups = 1;
+    for (int64_t first = 0; block <= 16 && first < kmax; first += block) {
+        const int64_t groups = m - first <= mfk::lu_panel_max_rows() ? mfk::lu_panel_workgroups(m - first) : 0;
+        if (groups <= 2 * cus) panel_groups = std::max(panel_groups, groups);
+    }
+    mfk::WaitingPlaces places;
+    if (panel_groups > 1 && !places.take(h->device, {panel_groups, 2, cus})) panel_groups = 1;
     double *pbuf = (double *)grow_panels(h, mfk::lu_panel_doubles() * sizeof(double));
     if (!pbuf) return fail(MFLA_ERR_HIP, "scratch allocation failed");
     HIPCHK(mfk::zero_fill(1, s, (int64_t)mfk::lu_panel_doubles(), 1, DV{pbuf, 1, 0, 0}));
@@ -1211,8 +1221,8 @@ static int sytrf_run(mfla_handle h, int N, const mfla_matrix &A, const mfla_matr
         // below the panel (at most the MFLA_LDLT_PANEL_WORKGROUPS cap) when
         // the weighted-panel buffer holds its keep sets and partials
         const bool grid_fits = mfk::ldlt_panel_grid_doubles(N, n) <= half;
-        const int64_t gcap = ldlt_panel_workgroup_cap();
-        const bool use_grid = grid_fits && gcap > 0;     // its panels also write the weighted rows
+        const int64_t cus = stream_cus(h, s), gcap = std::min(ldlt_panel_workgroup_cap(), cus);
+        bool use_grid = grid_fits && gcap > 0;           // its panels also write the weighted rows
         auto workgroups = [&](int64_t pf) { return std::max<int64_t>(1, std::min(gcap, mfk::cdiv(n - pf - 1, kLdltPanelRows))); };
         // Look-ahead: while it splits, the panels run on a stream confined to
         // a few CUs and each panel's trailing update is cut in three: the
@@ -1236,13 +1246,17 @@ static int sytrf_run(mfla_handle h, int N, const mfla_matrix &A, const mfla_matr
         if (la) {
             if (ensure_side(h) != hipSuccess || ensure_la_streams(h, kLdltPanelCUs) != hipSuccess) { (void)hipGetLastError(); la = false; }
         }
+        if (W && avail < 3 * half) la = false;
+        // the panels' workgroups wait for each other, one a CU: on the panel
+        // stream's CUs, else on the call's, else panels of one workgroup
+        mfk::WaitingPlaces places;
+        if (la) la = places.take(h->device, {g0, 1, std::min<int64_t>(kLdltPanelCUs, cus)});
+        if (!la && g0 > 1) use_grid = places.take(h->device, {g0, 1, cus});
         if (!W) {
             const size_t len = (la ? 3 : 1) * half;
             if (hipMalloc(&W, sizeof(double) * len) != hipSuccess) return fail(MFLA_ERR_HIP, "weighted panel allocation failed");
             own = true;
-            avail = len;
         }
-        if (avail < 3 * half) la = false;
         hipStream_t ps = s, us = s;                      // while splitting: panels, trailing updates
         // `to` waits for the work launched on `from` so far
         auto order = [&](hipStream_t from, hipStream_t to, hipEvent_t ev) -> hipError_t {

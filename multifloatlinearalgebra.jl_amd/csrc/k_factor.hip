@@ -516,9 +516,11 @@ __global__ __launch_bounds__(256, 8) void k_lu_scale_update(DV A, int64_t k, int
 // beside it, every column. Tags hold the column's number + 1; the two buffers
 // alternate, and a workgroup writes one again only after every workgroup has
 // published the column in between, i.e. has read it. The G workgroups need
-// not start together, only to be resident together in the end (at most 128 on
-// the chip's 256 CUs, whatever runs beside them ends by itself); a wait is bounded
-// all the same: past it st->info = kGridTimeout and the call fails.
+// not start together, only to be resident together in the end: whatever runs
+// beside them ends by itself except other waiting panels, and the caller runs
+// this kernel only where its CUs hold those and this one together
+// (WaitingPlaces). Another process's panels it cannot see, so a wait is
+// bounded: past it st->info = kGridTimeout and the call fails.
 constexpr int LU_B = 16, LU_MAXG = 128, LU_SLOT = 72;   // slot: N limbs, row, (at 8) 16 N values
 constexpr int64_t kGridTimeout = -2;      // st->info after a bounded wait ended
 
