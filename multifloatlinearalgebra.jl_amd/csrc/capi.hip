@@ -1221,7 +1221,7 @@ static int sytrf_run(mfla_handle h, int N, const mfla_matrix &A, const mfla_matr
         // below the panel (at most the MFLA_LDLT_PANEL_WORKGROUPS cap) when
         // the weighted-panel buffer holds its keep sets and partials
         const bool grid_fits = mfk::ldlt_panel_grid_doubles(N, n) <= half;
-        const int64_t cus = stream_cus(h, s), gcap = std::min(ldlt_panel_workgroup_cap(), cus);
+        const int64_t cus = stream_cus(h, s), gcap = std::min(ldlt_panel_workgroup_cap(), cus / mfk::kXcds * mfk::kXcds);
         bool use_grid = grid_fits && gcap > 0;           // its panels also write the weighted rows
         auto workgroups = [&](int64_t pf) { return std::max<int64_t>(1, std::min(gcap, mfk::cdiv(n - pf - 1, kLdltPanelRows))); };
         // Look-ahead: while it splits, the panels run on a stream confined to

@@ -22,17 +22,22 @@ struct WaitingCall {
     int64_t groups, per_cu, cus;
 };
 
-// Whether every call's launches end: one does if its CUs hold everybody's
-// waiting workgroups together, all of them taken to be on those CUs; once it
-// has ended, its places are free for the rest. A workgroup that needs a whole
-// CU counts each of the others as a whole one too.
+// Workgroups are dealt to the eight XCDs in turn whatever room each has, so
+// the first XCD's share is what has to fit its CUs (three 9-workgroup panels
+// put six workgroups on the four CUs a 32-CU mask has there).
+constexpr int64_t kXcds = 8;
+
+// Whether every call's launches end: one does if an XCD's CUs hold everybody's
+// share of waiting workgroups together, all of them taken to be on those CUs;
+// once it has ended, its places are free for the rest. A workgroup that needs
+// a whole CU counts each of the others as a whole one too.
 inline bool waiting_calls_end(std::vector<WaitingCall> calls) {
     for (bool ended = true; ended && !calls.empty();) {
         ended = false;
         for (size_t i = 0; i < calls.size() && !ended; ++i) {
             double need = 0.0;
-            for (const WaitingCall &c : calls) need += (double)c.groups / (calls[i].per_cu == 1 ? 1 : c.per_cu);
-            if (need <= (double)calls[i].cus) {
+            for (const WaitingCall &c : calls) need += (double)((c.groups + kXcds - 1) / kXcds) / (calls[i].per_cu == 1 ? 1 : c.per_cu);
+            if (need <= (double)(calls[i].cus / kXcds)) {
                 calls.erase(calls.begin() + (std::ptrdiff_t)i);
                 ended = true;
             }

@@ -47,6 +47,10 @@ def takes(tmp_path_factory):
     # on one 32-CU mask a single panel of 64, and again once it has ended
     (["0:64:2:32", "0:64:2:32", "-", "0:64:2:32"], "101"),
     (["0:65:2:32", "0:64:2:32"], "01"),
+    # nine workgroups are two on the first XCD, whose share of the mask is four CUs
+    (["0:9:1:32"] * 3, "110"),
+    (["0:8:1:32"] * 5, "11110"),
+    (["0:16:2:8", "0:17:2:8", "0:2:2:7"], "100"),
     # ldlt!'s panels, one a CU, all on the same 32 CUs; on the device's CUs instead
     (["0:32:1:32", "0:32:1:32", "0:32:1:256"], "101"),
     (["0:64:1:256"] * 5, "11110"),
