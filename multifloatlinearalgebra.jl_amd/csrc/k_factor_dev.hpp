@@ -144,9 +144,13 @@ __device__ void wg_argmax_lead(mf::V<N> &val, int64_t &idx, double *sv_buf, int6
 }
 
 // ------------------------------------------------------------------ LDLT
-// ldlt.jl:65-101 (scaled 2x2 elimination)
+// ldlt.jl:65-101 (scaled 2x2 elimination). Inlined by force: with its seven
+// four-limb divisions unrolled the compiler makes it a function, and the
+// kernels that call it pass everything through scratch (240 to 400 bytes a lane;
+// Float64x4 ldlt!, unblocked, n = 100 / 300: 3.33 / 24.9 ms as a function, 2.85
+// / 23.3 inlined; 1000 systems of 16 to 256 in a batch 34.9 against 33.8).
 template <int N>
-__device__ bool solve2x2(const mf::V<N> &d11, const mf::V<N> &d21, const mf::V<N> &d22, const mf::V<N> &f, const mf::V<N> &s,
+__device__ __forceinline__ bool solve2x2(const mf::V<N> &d11, const mf::V<N> &d21, const mf::V<N> &d22, const mf::V<N> &f, const mf::V<N> &s,
                          mf::V<N> &x1, mf::V<N> &x2) {
     mf::V<N> scale = mf::vmax(mf::vmax(mf::vabs(d11), mf::vabs(d21)), mf::vabs(d22));
     x1 = mf::zero<N>(); x2 = mf::zero<N>();
