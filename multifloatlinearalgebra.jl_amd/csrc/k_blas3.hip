@@ -27,7 +27,7 @@
 
 namespace mfk {
 
-template <int N, int NET, int TM, int TN, int BK, int MODE, bool LOWER>
+template <int N, int NET, int TM, int TN, int BK, int MODE, bool LOWER, bool AHEAD>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 8))) void k_tile(int64_t n, int64_t K, DV A, DV B, DV C, S<N> alpha, S<N> beta,
                                               int beta_zero, int64_t row_lo, int64_t row_hi, const Status *status,
                                               int64_t status_limit, int swap) {
@@ -216,12 +216,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 8))) voi
                     else acc[a][b] = mf::Mac<N, NET>::apply(acc[a][b], av[a], bv[b]);
                 }
         };
-        if constexpr (TM * TN == 1 && MODE == MODE_AB && !LOWER) {
-            // one element a thread: the next k's operands are read while this
-            // one's product is summed, two k a turn (a wave alone on its SIMD
-            // otherwise waits for LDS at every k: x4 256^3 148 -> 142 us, 100 x
-            // 300 x 100 174 -> 160; the triangular solves' updates, four waves on
-            // a SIMD, lose by the registers: x4 4096 x 256 18.9 -> 20.0 ms)
+        if constexpr (AHEAD) {
+            // the next k's operands are read while this one's product is
+            // summed, two k a turn (pick() says where)
             mf::V<N> a0[TM], b0[TN], a1[TM], b1[TN];
             read(0, a0, b0);
             int kk = 0;
@@ -259,12 +256,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 8))) voi
 }
 
 // ---------------------------------------------------------------- launcher
-template <int N, int NET, int TM, int TN, int BK, int MODE, bool LOWER>
+template <int N, int NET, int TM, int TN, int BK, int MODE, bool LOWER, bool AHEAD = false>
 static hipError_t go(hipStream_t s, int64_t rows, int64_t n, int64_t K, const DV &A, const DV &B, const DV &C,
                      const S<N> &al, const S<N> &be, int bz, int64_t row_lo, const Status *st, int64_t lim, int swap) {
     constexpr int BM = 16 * TM, BN = 16 * TN;
     dim3 grid((unsigned)cdiv(rows, BM), (unsigned)cdiv(n, BN));
-    hipLaunchKernelGGL((k_tile<N, NET, TM, TN, BK, MODE, LOWER>), grid, dim3(256), 0, s, n, K, A, B, C, al, be, bz, row_lo,
+    hipLaunchKernelGGL((k_tile<N, NET, TM, TN, BK, MODE, LOWER, AHEAD>), grid, dim3(256), 0, s, n, K, A, B, C, al, be, bz, row_lo,
                        row_lo + rows, st, lim, swap);
     return hipGetLastError();
 }
@@ -283,6 +280,21 @@ static hipError_t pick(hipStream_t s, int tile, int64_t rows, int64_t n, int64_t
     }
     if (tile == 2 || tile == 3) return go<N, NET, 2, 4, 16, MODE, LOWER>(s, rows, n, K, A, B, C, al, be, bz, row_lo, st, lim, swap);
     if (tile == 1) return go<N, NET, 2, 2, 16, MODE, LOWER>(s, rows, n, K, A, B, C, al, be, bz, row_lo, st, lim, swap);
+    // One element a thread: a wave alone on its SIMD waits for LDS at every k
+    // unless it reads ahead, which costs registers (x3 62 -> 87 of them, 8 -> 5
+    // waves a SIMD). Read ahead, us: 256^3 x4 145.5 -> 133.7, x3 64.3 -> 60.4,
+    // x2 30.4 -> 28.6; 100 x 300 x 100 x4 173.8 -> 159.3, x3 83.6 -> 76.0. With
+    // 4096 workgroups and more, sixteen on a CU, the waves hide it themselves:
+    // 4096 x 16 x 4096 x2 and x3 within 1 %, x4 1867 -> 1885 and 2048 x 16 x 2048
+    // x4 464 -> 471 (so not there; x2 and x3 keep it for lu!, whose panels
+    // beside such an update gain by its fewer waves: x3 n = 1999 24.2 -> 21.8
+    // ms). One limb loses everywhere it differs (2048 x 16 x 2048 30.8 -> 35.2,
+    // 100 x 300 x 100 20.2 -> 22.5), and so do the triangular solves' updates
+    // (x4 4096 x 256 18.9 -> 20.0 ms).
+    if constexpr (MODE == MODE_AB && !LOWER && N > 1) {
+        if (N < 4 || cdiv(rows, 16) * cdiv(n, 16) < 4096)
+            return go<N, NET, 1, 1, 16, MODE, LOWER, true>(s, rows, n, K, A, B, C, al, be, bz, row_lo, st, lim, swap);
+    }
     return go<N, NET, 1, 1, 16, MODE, LOWER>(s, rows, n, K, A, B, C, al, be, bz, row_lo, st, lim, swap);
 }
 
