@@ -36,8 +36,11 @@ def test_panel_edges(oracle, N, m, n):
         assert check(oracle, rand_mf(rng, N, m, n), block=5) == 0
 
 
-# 128 workgroups of 16 rows, then two and four rows a thread, then column kernels
-@pytest.mark.parametrize("N,m", [(2, 2048), (2, 2049), (4, 2060), (3, 4096), (2, 4097), (4, 4110), (2, 8192), (2, 8193)])
+# one row a thread up to 1024 rows (64 workgroups), two up to 2048, four up to
+# 8192, then column kernels; 1040 and 2060 cross an edge between panels
+@pytest.mark.parametrize("N,m", [(2, 2048), (2, 2049), (4, 2060), (3, 4096), (2, 4097), (4, 4110), (2, 8192), (2, 8193),
+                                 (2, 1024), (3, 1024), (4, 1024), (2, 1025), (3, 1025), (4, 1025), (2, 1040), (3, 1040), (4, 1040), (3, 1700),
+                                 (3, 2049), (4, 8192)])
 def test_tall_panels(oracle, N, m):
     rng = np.random.default_rng(case_seed(N, m))
     assert check(oracle, rand_mf(rng, N, m, 37), threads=8) == 0
