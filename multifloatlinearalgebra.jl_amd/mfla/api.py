@@ -109,7 +109,9 @@ _ORDER = {"auto": 0, "exact": 1, "blocked": 2}
 @dataclass
 class KernelConfig:
     """KernelConfig (src/types.jl:13-27) plus the device-only knobs
-    ``trsm_order`` (backward-substitution order) and ``gemm_tile``."""
+    ``trsm_order`` (backward-substitution order) and ``gemm_tile``. "auto" order
+    is MFLA's exact one up to n = 256 and the blocked one beyond; the adjoints'
+    solves (solve_adjoint, logdet_adjoint) take it as "blocked" at every n."""
 
     reduction_tile: int = 64
     column_tile: int = 16

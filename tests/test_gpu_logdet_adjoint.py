@@ -39,3 +39,24 @@ def test_inverse_at_block_edges(oracle, N, n):
     assert np.max(np.abs(err) / scale) <= 64 * n * eps(N)
     half = AD.logdet_adjoint(F, one * 0.5).cpu().numpy()
     assert np.array_equal(half, G * 0.5)
+
+
+@pytest.mark.parametrize("N,n", [(2, 70), (4, 130), (3, 256)])
+def test_solve_adjoint_keeps_a_stated_order(oracle, N, n):
+    """"exact" and "blocked" give the bits of a solve in that order; the order
+    left open is the blocked one, also at n <= 256."""
+    import mfla as M
+    from mfla import autodiff as AD
+
+    rng = np.random.default_rng(case_seed("order", N, n))
+    R = rand_mf(rng, N, n, n)
+    S = np.zeros((N, n, n))
+    oracle.gemm(S, R, np.ascontiguousarray(np.transpose(R, (0, 2, 1))), fused=False)
+    S[0, np.arange(n), np.arange(n)] += n
+    F = M.cholesky_(torch.from_numpy(S).cuda())
+    X, Xbar = torch.from_numpy(rand_mf(rng, N, n, 3)).cuda(), torch.from_numpy(rand_mf(rng, N, n, 3)).cuda()
+    solved = {o: M.solve(F, Xbar, config=M.KernelConfig(trsm_order=o)).cpu().numpy() for o in ("exact", "blocked")}
+    assert not np.array_equal(solved["exact"], solved["blocked"])
+    for order, want in (("exact", "exact"), ("blocked", "blocked"), ("auto", "blocked")):
+        Bbar, _ = AD.solve_adjoint(F, X, Xbar, config=M.KernelConfig(trsm_order=order))
+        assert np.array_equal(Bbar.cpu().numpy(), solved[want]), order
