@@ -54,6 +54,7 @@ def test_noalloc_ldlt_failure_state_equals_sytrf():
 
     rng = np.random.default_rng(77)
     for n, zero in ((600, 333), (200, 50)):
+        print(f"noalloc ldlt failure x4 n={n}", flush=True)
         A = symmetric_indefinite(rng, 4, n)
         A[:, zero, :] = 0.0
         A[:, :, zero] = 0.0
