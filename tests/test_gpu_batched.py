@@ -7,7 +7,7 @@ import numpy as np
 import pytest
 import torch
 
-from mfutil import HELD_OFF_GPU, assert_bitwise, eps, rand_mf
+from mfutil import assert_bitwise, eps, rand_mf
 
 pytestmark = pytest.mark.gpu
 
@@ -135,7 +135,6 @@ def test_batched_orders_91_to_256_systolic(oracle):
         assert (r["blocks"] == 2).any()
 
 
-@HELD_OFF_GPU
 def test_batched_orders_91_to_256_exact_backward(oracle):
     """The same systems with MFLA's exact backward order: X bitwise."""
     from mfla.batched import Batch

@@ -9,7 +9,7 @@ import numpy as np
 import pytest
 import torch
 
-from mfutil import HELD_OFF_GPU, assert_bitwise, eps, rand_mf, case_seed
+from mfutil import assert_bitwise, eps, rand_mf, case_seed
 
 pytestmark = pytest.mark.gpu
 
@@ -80,7 +80,7 @@ def test_gemm_matches_oracle(mfla, oracle, N, shape):
             assert_bitwise(host(Cd), ref, f"x{N} {shape} {strat}")
 
 
-@pytest.mark.parametrize("N", [1, 2, pytest.param(3, marks=HELD_OFF_GPU), 4])
+@pytest.mark.parametrize("N", [1, 2, 3, 4])
 def test_gemm_tile_shapes_bitwise_identical(mfla, oracle, N):
     """Every tile shape (16x16, 32x32, 32x64, 64x64) gives MFLA's bits. 131
     rows: for x3 the fused route runs mulacc_x3 on rows 0..127 and the

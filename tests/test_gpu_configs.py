@@ -21,7 +21,7 @@ import numpy as np
 import pytest
 import torch
 
-from mfutil import HELD_OFF_GPU, assert_bitwise, eps
+from mfutil import assert_bitwise, eps
 
 pytestmark = pytest.mark.gpu
 
@@ -224,7 +224,6 @@ def test_batched_config3_sample(mfla, oracle):
         check_solution_residual(oracle, N, kind, A, B, r["X"])
 
 
-@HELD_OFF_GPU
 def test_batched_config3_sample_exact_backward(mfla, oracle):
     """The same sample with MFLA's exact backward order: X bitwise."""
     from mfla.batched import Batch
