@@ -174,8 +174,9 @@ def bench_ozaki(args, M, torch, g):
     e1.record()
     torch.cuda.synchronize()
     ms = e0.elapsed_time(e1) / steps
-    S = {1: 11, 2: 19, 3: 27, 4: 34}[N]
-    ops = 2.0 * (S + 1) * (S + 2) / 2 * n * n * ((n + 127) // 128 * 128)
+    from mfla.suite import int8_pairs
+
+    ops = 2.0 * int8_pairs(N, n) * n * n * ((n + 63) // 64 * 64)
     return {"ms": round(ms, 3), "speedup_vs_eft_gemm": round(g["ms"] / ms, 2),
             "int8_tops": round(ops / (ms * 1e-3) / 1e12, 1), "int8_frac_of_5pops": round(ops / (ms * 1e-3) / 5.0e15, 4),
             "x_equiv_tflops": round(float(n) ** 3 * network_cost(N)[0] / (ms * 1e-3) / 1e12, 2),

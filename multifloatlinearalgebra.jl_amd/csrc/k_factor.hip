@@ -1702,8 +1702,12 @@ template <int N> static S<N> mk(const double *v) { S<N> s; for (int l = 0; l < N
 
 size_t chol_step_doubles(int N, int64_t n) { return (size_t)N * n * CS_B; }
 
-// Rows per wave: 4, or 8 from 3072 rows on (a workgroup per CU either way, so
-// that no two diagonal waves share a SIMD).
+// Rows per wave: 4, or 8 from 3072 rows on, so that up to 6144 rows there is at
+// most a workgroup per CU and no two diagonal waves share a SIMD. Beyond, some
+// do, beside trailing updates that take far longer: against the three kernels a
+// panel took before, n = 8192, x1 39.8 -> 37.8 ms, x2 116.8 -> 115.1, x4 687.3 ->
+// 687.1, x3 345.6 -> 347.3 (0.5 %, as two runs differ); 12 or 16 rows a wave there
+// measured the same (x3 347.1, x4 688.9).
 hipError_t chol_step(int N, hipStream_t s, const DV &A, int64_t n, int64_t first, int nb, int np, double *diag, Status *st) {
     if (nb < 1 || nb > CS_B || np < 0 || np > CS_B || first < np) return hipErrorInvalidValue;
     const int64_t rest = n - first - nb;

@@ -495,7 +495,12 @@ hipError_t oz_round_fp64(hipStream_t s, int64_t K, int64_t ncols, const DV &D, c
 // share one block below (0.097 / 0.601 / 4.65 / 37.9, but four times the
 // workgroups). Fewer limbs share one block at every size (x3 0.049 / 0.284 /
 // 2.08 / 17.8 against 0.055 / 0.334 / 2.21 / 19.6 for two, x2 0.029 / 0.177 /
-// 1.34 / 11.5 against 0.033 / 0.224 / 1.60 / 15.1).
+// 1.34 / 11.5 against 0.033 / 0.224 / 1.60 / 15.1). The four-limb two-block
+// shape spills 19 registers, 80 bytes a lane, and is the faster one all the
+// same; with two blocks of three limbs' 27 digits nothing spills, and A's digits
+// are read half as often (whole gemm!, 512 x 8192 x 512 1.12 against 1.81 ms, 2000
+// x 6000 x 1000 5.03 against 8.65, 4096 x 4160 x 4096 26.0 against 52.0; 300 x 5000
+// x 70 0.383 against 0.380).
 template <int N, int B, int S, int KS, int WN, int AHEAD, int EARLY>
 static hipError_t oz_launch(hipStream_t s, int64_t m, int64_t n, int64_t K, const int8_t *dA, const int8_t *dB, const int *ea, const int *eb,
                             const DV &C, const double *alpha, const double *beta, int beta_zero) {
@@ -522,7 +527,7 @@ hipError_t oz_gemm(int N, hipStream_t s, int64_t m, int64_t n, int64_t K, int S,
         case 17: OZ_GO(2, 8, 17, 4, 1, 8, 6);
         case 10: OZ_GO(1, 8, 10, 4, 1, 4, 4);
         case 34: OZ_GO(4, 7, 34, 4, 1, 8, 6);
-        case 27: OZ_GO(3, 7, 27, 4, 2, 6, 6);   // one block: 8.6 ms for 2000 x 6000 x 1000
+        case 27: OZ_GO(3, 7, 27, 4, 2, 6, 6);
         case 19: OZ_GO(2, 7, 19, 4, 1, 8, 6);
         case 11: OZ_GO(1, 7, 11, 4, 1, 4, 5);
     }

@@ -86,6 +86,14 @@ def _memory(name, N, bytes_, macs, t, **extra):
     return r
 
 
+def int8_pairs(N, k):
+    """Digit pairs gemm!'s INT8 products form per output and reduction step:
+    all (s, t) with s + t <= S of S digits (8 bits each while the padded
+    reduction is at most 4096, 7 beyond)."""
+    S = ({1: 10, 2: 17, 3: 24, 4: 30} if (k + 63) // 64 * 64 <= 4096 else {1: 11, 2: 19, 3: 27, 4: 34})[N]
+    return S * (S + 1) // 2 + S - 1
+
+
 def case_gemm(N, m, k, n, reps=2, strategy="auto"):
     A, B = rand_dev(N, m, k, 1), rand_dev(N, k, n, 2)
     C = torch.zeros((N, n, m), dtype=torch.float64, device="cuda")
@@ -93,9 +101,7 @@ def case_gemm(N, m, k, n, reps=2, strategy="auto"):
     t = _time(lambda: M.gemm_(C, A, B, config=cfg), reps)
     if strategy == "ozaki":
         # INT8 matrix-core work: digit-pair products over K per output
-        S = {1: 11, 2: 19, 3: 27, 4: 34}[N]
-        pairs = (S + 1) * (S + 2) // 2
-        ops = 2.0 * pairs * m * n * ((k + 63) // 64 * 64)
+        ops = 2.0 * int8_pairs(N, k) * m * n * ((k + 63) // 64 * 64)
         return {"case": f"gemm {m}x{k}x{n} (ozaki)", "limbs": N, "ms": round(t * 1e3, 3), "macs": m * k * n,
                 "x_equiv_tflops": round(m * k * n * F_N[N] / t / 1e12, 3), "int8_tops": round(ops / t / 1e12, 1),
                 "int8_frac": round(ops / t / 5.0e15, 4)}
