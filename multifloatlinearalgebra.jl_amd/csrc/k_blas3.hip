@@ -27,7 +27,7 @@
 
 namespace mfk {
 
-template <int N, int NET, int TM, int TN, int BK, int MODE, bool LOWER, bool AHEAD>
+template <int N, int NET, int TM, int TN, int BK, int MODE, bool LOWER, bool AHEAD>   // AHEAD: TM = TN = 1, MODE_AB
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 8))) void k_tile(int64_t n, int64_t K, DV A, DV B, DV C, S<N> alpha, S<N> beta,
                                               int beta_zero, int64_t row_lo, int64_t row_hi, const Status *status,
                                               int64_t status_limit, int swap) {
@@ -197,7 +197,28 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 8))) voi
             }
         }
         const int kend = (K - k0) < BK ? (int)(K - k0) : BK;
-        auto read = [&](int kk, mf::V<N> (&av)[TM], mf::V<N> (&bv)[TN]) {
+        if constexpr (AHEAD) {
+            // the next k's operands are read while this one's product is
+            // summed, two k a turn (pick() says where)
+            auto read = [&](int kk, mf::V<N> &av, mf::V<N> &bv) {
+#pragma unroll
+                for (int l = 0; l < N; ++l) av.x[l] = As[a_slot(kk, tx, l)];
+#pragma unroll
+                for (int l = 0; l < N; ++l) bv.x[l] = Bs[b_slot(kk, ty) + l];
+            };
+            mf::V<N> a0, b0, a1, b1;
+            read(0, a0, b0);
+            int kk = 0;
+            for (; kk + 1 < kend; kk += 2) {
+                read(kk + 1, a1, b1);
+                acc[0][0] = mf::Mac<N, NET>::apply(acc[0][0], a0, b0);
+                read(kk + 2 < BK ? kk + 2 : BK - 1, a0, b0);
+                acc[0][0] = mf::Mac<N, NET>::apply(acc[0][0], a1, b1);
+            }
+            if (kk < kend) acc[0][0] = mf::Mac<N, NET>::apply(acc[0][0], a0, b0);
+        } else
+        for (int kk = 0; kk < kend; ++kk) {
+            mf::V<N> av[TM], bv[TN];
 #pragma unroll
             for (int a = 0; a < TM; ++a)
 #pragma unroll
@@ -206,8 +227,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 8))) voi
             for (int b = 0; b < TN; ++b)
 #pragma unroll
                 for (int l = 0; l < N; ++l) bv[b].x[l] = Bs[b_slot(kk, ty * TN + b) + l];
-        };
-        auto step = [&](const mf::V<N> (&av)[TM], const mf::V<N> (&bv)[TN]) {
 #pragma unroll
             for (int a = 0; a < TM; ++a)
 #pragma unroll
@@ -215,26 +234,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 8))) voi
                     if (MODE == MODE_SUB) acc[a][b] = swap ? mf::msub(acc[a][b], bv[b], av[a]) : mf::msub(acc[a][b], av[a], bv[b]);
                     else acc[a][b] = mf::Mac<N, NET>::apply(acc[a][b], av[a], bv[b]);
                 }
-        };
-        if constexpr (AHEAD) {
-            // the next k's operands are read while this one's product is
-            // summed, two k a turn (pick() says where)
-            mf::V<N> a0[TM], b0[TN], a1[TM], b1[TN];
-            read(0, a0, b0);
-            int kk = 0;
-            for (; kk + 1 < kend; kk += 2) {
-                read(kk + 1, a1, b1);
-                step(a0, b0);
-                read(kk + 2 < BK ? kk + 2 : BK - 1, a0, b0);
-                step(a1, b1);
-            }
-            if (kk < kend) step(a0, b0);
-        } else {
-            for (int kk = 0; kk < kend; ++kk) {
-                mf::V<N> av[TM], bv[TN];
-                read(kk, av, bv);
-                step(av, bv);
-            }
         }
         __syncthreads();
     }
