@@ -132,9 +132,9 @@ __global__ __launch_bounds__(256, N == 4 ? 5 : 8) void k_trsm_diag_wave(int64_t 
 // through LDS: the workgroup's four waves share them, CH columns at a time,
 // the next CH loading into registers meanwhile. A step is one division and one
 // product (x2 0.3 us, x4 1.9), and a coefficient loaded one step ahead by each
-// wave made it wait for memory instead (a 4096-unknown solve, x2 256 right-hand sides
-// 4.41 -> 3.81 ms, x2 64 backward 3.75 -> 3.14, x4 64 backward 12.4 -> 11.9, x4
-// 64 forward 11.8 -> 10.9 with the faster division, x3 and x4 256 unchanged).
+// wave made it wait for memory instead (a 4096-unknown solve, x2 256 right-hand
+// sides 4.41 -> 3.81 ms, x2 64 backward 3.75 -> 3.14, x4 64 backward 12.4 -> 11.9,
+// x3 256 10.0 -> 9.7 both ways). Four limbs' forward solves take k_trsm_diag_mem.
 //
 // With K > 0 the kernel first subtracts the K <= 64 terms of the block solved
 // just before (unknowns q0 .. q0 + K - 1, ascending q: the order and operations
@@ -225,6 +225,62 @@ __global__ __launch_bounds__(256, N == 4 ? 4 : 6) void k_trsm_diag_lds(int64_t p
     solve_end<N>(v, valid, X, p, c);
 }
 
+// The same for four limbs' forward solves, each wave loading its coefficients
+// from memory at the top of the step and no barrier in the loop: the chunks'
+// staging and barriers cost more than they hide there (64 x 64 183 -> 159 us,
+// 192 x 16 571 -> 492, 300 x 100 985 -> 855, 1000 x 100 3.23 -> 2.92 ms, 4096 x 128
+// 14.65 -> 14.24, 4096 x 256 19.4 -> 18.9). Backward the chunks are the faster
+// form or equal (300 x 100 877 against 916 us, 250 x 1000 765 against 817), and with
+// three limbs both ways (4096 x 256 9.73 against 10.0 ms, 9.95 against 10.4).
+__global__ __launch_bounds__(256, 5) void k_trsm_diag_mem(int64_t p0, int nbk, int64_t nrhs, DV X, DV CA, DV D, int unit, int swap, const Status *st,
+                                                          int64_t lim, int64_t q0, int K, const unsigned *far_flag, unsigned far_wait,
+                                                          unsigned *err, unsigned *start_sig, unsigned start_value) {
+    constexpr int N = 4;
+    __builtin_amdgcn_s_setprio(3);
+    mark_start(start_sig, start_value);
+    if (st && st->info != 0 && (lim == 0 || st->info < 0 || st->info <= lim)) return;
+    const bool ok = far_flag == nullptr || wait_flag(far_flag, far_wait);
+    __shared__ __align__(16) double dg[TB * N];
+    const int t = threadIdx.x, lane = t & 63;
+    const int64_t c = (int64_t)blockIdx.x * 4 + (t >> 6), cc = c < nrhs ? c : nrhs - 1;
+    const bool valid = lane < nbk && c < nrhs;
+    const int64_t p = p0 + lane, pc = p0 + (lane < nbk ? lane : nbk - 1);   // pc: in bounds for every lane
+    if (!unit && t < nbk) lds_put<N>(&dg[t * N], ld<N>(D, p0 + t, p0 + t));
+    mf::V<N> v = valid ? ld<N>(X, p, c) : mf::zero<N>();
+    if (!ok) {
+#pragma unroll
+        for (int l = 0; l < N; ++l) v.x[l] = __builtin_nan("");
+        if (t == 0) __hip_atomic_store(err, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    if (K > 0) {
+        mf::V<N> an = ld<N>(CA, pc, q0), xn = ld<N>(X, q0, cc);
+        for (int k = 0; k < K; ++k) {
+            const mf::V<N> a = an, xq = xn;
+            if (k + 1 < K) {
+                an = ld<N>(CA, pc, q0 + k + 1);
+                xn = ld<N>(X, q0 + k + 1, cc);
+            }
+            v = swap ? mf::msub(v, xq, a) : mf::msub(v, a, xq);
+        }
+    }
+    __syncthreads();
+    for (int s = 0; s < nbk; ++s) {
+        const mf::V<N> a = ld<N>(CA, pc, p0 + s);
+        mf::V<N> xq;
+#pragma unroll
+        for (int l = 0; l < N; ++l) xq.x[l] = group_bcast<64>(v.x[l], 0, s);
+        if (!unit) xq = mf::div(xq, lds_get<N>(&dg[s * N]));
+        if (valid) {
+            if (lane == s) {
+                v = xq;
+                stv<N>(X, p0 + s, c, xq);
+            } else if (lane > s) {
+                v = swap ? mf::msub(v, xq, a) : mf::msub(v, a, xq);
+            }
+        }
+    }
+}
+
 // Forward look-ahead with the next block's rows streamed. A workgroup of 8
 // waves takes 4 right-hand sides: waves 0-3 solve the block (the operations
 // of k_trsm_diag_wave with one wave per right-hand side and no previous-block
@@ -238,7 +294,7 @@ __global__ __launch_bounds__(256, N == 4 ? 4 : 6) void k_trsm_diag_lds(int64_t p
 // the wait ends; it is bounded all the same, and past the bound the rows
 // are written as NaN (and *err = 1) instead of values without the update.
 constexpr int kStreamRhs = 4;
-template <int N>
+template <int N, bool SEL>
 __global__ __launch_bounds__(512, N == 4 ? 3 : 4) void k_trsm_diag_stream(int64_t p0, int nbk, int64_t p1, int nn, int64_t nrhs, DV X,
                                                                         DV CA, DV D, int unit, int swap, const Status *st, int64_t lim,
                                                                         const unsigned *far_flag, unsigned far_wait, unsigned *err,
@@ -281,9 +337,18 @@ __global__ __launch_bounds__(512, N == 4 ? 3 : 4) void k_trsm_diag_stream(int64_
                 lds_put<N>(&xs[(r * 64 + s) * N], xq);
                 __hip_atomic_store(&cnt[r], s + 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
             }
-            solve_step<N>(v, xq, a, swap, valid, lane == s, lane > s, X, q, c);
+            if constexpr (SEL) {
+                solve_step<N>(v, xq, a, swap, valid, lane == s, lane > s, X, q, c);
+            } else if (valid) {   // solve_step's branches, here: as a call they took x4 4096 x 64 from 10.95 to 11.25 ms
+                if (lane == s) {
+                    v = xq;
+                    stv<N>(X, q, c, xq);
+                } else if (lane > s) {
+                    v = swap ? mf::msub(v, xq, a) : mf::msub(v, a, xq);
+                }
+            }
         }
-        solve_end<N>(v, valid, X, p, c);
+        if constexpr (SEL) solve_end<N>(v, valid, X, p, c);
     } else {
         const bool valid = lane < nn && c < nrhs;
         const int64_t p = p1 + lane, pc = p1 + (lane < nn ? lane : nn - 1);
@@ -435,11 +500,14 @@ static hipError_t diag(hipStream_t s, bool fwd, int64_t p0, int nbk, int64_t nrh
     if (nbk < 1 || nbk > TB || K < 0 || K > TB) return hipErrorInvalidValue;
     if (nbk > 32 || K > 0 || far_flag || start_sig) {
         const dim3 grid((unsigned)cdiv(nrhs, 4));
-        if (fwd)
-            hipLaunchKernelGGL((k_trsm_diag_lds<N, true>), grid, dim3(256), 0, s, p0, nbk, nrhs, X, CA, D, unit, swap, st, lim, q0, K, far_flag,
-                               far_wait, err, start_sig, start_value);
-        else
+        if (!fwd)
             hipLaunchKernelGGL((k_trsm_diag_lds<N, false>), grid, dim3(256), 0, s, p0, nbk, nrhs, X, CA, D, unit, swap, st, lim, q0, K, far_flag,
+                               far_wait, err, start_sig, start_value);
+        else if constexpr (N == 4)
+            hipLaunchKernelGGL(k_trsm_diag_mem, grid, dim3(256), 0, s, p0, nbk, nrhs, X, CA, D, unit, swap, st, lim, q0, K, far_flag, far_wait, err,
+                               start_sig, start_value);
+        else
+            hipLaunchKernelGGL((k_trsm_diag_lds<N, true>), grid, dim3(256), 0, s, p0, nbk, nrhs, X, CA, D, unit, swap, st, lim, q0, K, far_flag,
                                far_wait, err, start_sig, start_value);
         return hipGetLastError();
     }
@@ -534,8 +602,22 @@ static hipError_t solve_t(hipStream_t s, const TrsmArgs &a, const DV &X, const D
                 const int64_t p1 = p0 + nbk;
                 const int nn = (int)((n - p1) < TB ? (n - p1) : TB);
                 if (nn > 0) {
-                    hipLaunchKernelGGL(k_trsm_diag_stream<N>, dim3((unsigned)cdiv(nrhs, kStreamRhs)), dim3(512), 0, s, p0, nbk, p1, nn, nrhs, X,
-                                       CA, D, a.unit, a.swap_product, st, a.status_limit, a.far_flag, b, a.far_flag + 1, a.start_sig, b);
+                    auto stream = [&](auto sel) {
+                        hipLaunchKernelGGL((k_trsm_diag_stream<N, decltype(sel)::value>), dim3((unsigned)cdiv(nrhs, kStreamRhs)), dim3(512), 0, s, p0,
+                                           nbk, p1, nn, nrhs, X, CA, D, a.unit, a.swap_product, st, a.status_limit, a.far_flag, b, a.far_flag + 1,
+                                           a.start_sig, b);
+                    };
+                    // two limbs: selects shorten a step, but not where the side
+                    // stream's updates set the pace, and there they cost (selects /
+                    // branches, ms: 4096 x 8 2.74 / 2.96, 4096 x 16 2.84 / 2.97, 3000 x
+                    // 32 2.20 / 2.24, 1000 x 64 0.74 / 0.78; 4096 x 24 3.21 / 3.08, 3000
+                    // x 64 2.46 / 2.32, 4096 x 64 3.56 / 3.32; 2048 x 64 within 1 %)
+                    if constexpr (N == 2) {
+                        if (n * nrhs >= 96 * 1024) stream(std::false_type());
+                        else stream(std::true_type());
+                    } else {
+                        stream(std::integral_constant<bool, N < 4>());
+                    }
                     if ((r = hipGetLastError()) != hipSuccess) return r;
                 } else if ((r = diag<N>(s, true, p0, nbk, nrhs, X, CA, D, a.unit, a.swap_product, st, a.status_limit, 0, 0, nullptr, 0, nullptr,
                                         a.start_sig, b)) != hipSuccess) {
