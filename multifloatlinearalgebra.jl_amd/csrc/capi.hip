@@ -906,8 +906,9 @@ int mfla_potrf(mfla_handle h, int N, mfla_matrix A, int64_t *info, const mfla_co
     }
     // Panels of up to 16 columns: one kernel per panel (chol_step: the update
     // of its columns by the panel before, the panel, the rows below), the
-    // update of the columns beyond the next panel on the second stream.
-    if (block <= 16 && n > 0) {
+    // update of the columns beyond the next panel on the second stream. A single
+    // panel has neither and takes the panel kernel alone, without the store.
+    if (block <= 16 && n > block) {
         double *diag = (double *)grow_panels(h, mfk::chol_step_doubles(N, n) * sizeof(double));
         if (!diag) return fail(MFLA_ERR_HIP, "scratch allocation failed");
         const hipEvent_t updated[2] = {h->ev_update, h->ev_update2};   // by the panel's parity
