@@ -127,3 +127,43 @@ def test_ldlt_calls_at_once(N, calls):
     finally:
         for c in callers:
             c.close()
+
+
+def test_lu_beside_a_batch(oracle):
+    """lu!'s waiting panels beside a batch whose workgroups fill the device
+    and end by themselves."""
+    from mfla.batched import Batch
+
+    rng = np.random.default_rng(case_seed("lu beside a batch"))
+    N = 2
+    systems = []
+    for i in range(600):
+        n = 100 + i % 100
+        S = np.zeros((N, n, n))
+        G = rng.standard_normal((n, n))
+        S[0] = G @ G.T + n * np.eye(n)
+        systems.append((0, S, rng.standard_normal((N, 2, n)) * np.array([1.0, 2.0**-53])[:, None, None]))
+    A = rand_mf(rng, N, 1024, 40)
+    ref = A.copy()
+    info, ipiv = oracle.getrf(ref, 16, threads=8)[:2]
+    b = Batch(systems, N)
+    b.solve()
+    want = [r["A"].copy() for r in b.results()[:20]]
+    caller, q = Caller(ctypes.c_void_p(torch.cuda.Stream().cuda_stream)), torch.cuda.Stream()
+    try:
+        for rep in range(3):
+            Ad = torch.from_numpy(A).cuda()
+            b.restore()
+            torch.cuda.synchronize()
+            with torch.cuda.stream(q):
+                b.solve()
+            ipd = torch.empty(40, dtype=torch.int64, device="cuda")
+            om, inf = (ctypes.c_double * 4)(), ctypes.c_int64(-9)
+            rc = caller.lib.mfla_getrf(caller.h, N, caller.matrix(Ad), ipd.data_ptr(), om, ctypes.byref(inf), None, None)   # no wait for the batch
+            torch.cuda.synchronize()
+            same((caller.error(rc), inf.value, [Ad.cpu().numpy(), ipd.cpu().numpy()]), ("", info, [ref, ipiv]), "lu beside a batch")
+            for r, w in zip(b.results()[:20], want):
+                assert r["info"] == 0
+                assert_bitwise(r["A"], w, "batch beside lu")
+    finally:
+        caller.close()
